@@ -18,78 +18,117 @@ __global__ void k_fill(float *p, float v, size_t n)
 // gpu.c:104-115: C[i][j] = sum_k A[i][k] * B[k][j], a sequential fp32 sum
 // from 0.0f with k ascending and separately rounded products, so results are
 // bit-identical to the CPU backend.  A thread owns NC adjacent columns for MT
-// rows (a block-row of A, MT <= 16), so every B element is read once per MT
-// rows: the kernel streams B, which is what bounds it at small M (an LM head
-// reads K*N floats per token), and with NC = 4 a lane's B load is one 16-byte
-// word.  A is staged in LDS in chunks of MM_KC columns (every lane reads the
-// same words: broadcast); the MM_U B loads of a turn are issued before their
-// products.  Rows past M are zero in LDS and never stored.
+// rows; with RS = 2 the work group's upper two waves take the next MT rows of
+// the lower two's columns, whose B values they then find in the CU's cache.
+// A is staged in LDS in chunks of MM_KC columns (every lane reads the same
+// words: broadcast).  The rows of A for the next 4 k's are read from LDS, and
+// B's next MM_U loads issued, before the products of the current ones, so the
+// multiply and add per product are what is left to wait for.  Rows past M are
+// zero in LDS and never stored.
+//
+// What bounds it: HBM up to 4 rows (2.03 GB at K = 2048, N = 248,320: 325 us,
+// 6.3 TB/s), the vector issue slots above (16 rows: 254 M wave instructions,
+// 441 us).  Before, with one LDS read per product group right before its use,
+// 16 rows took 530-630 us there, and 16 / 4 / 1 rows at N = 32,768 took 293 /
+// 241 / 117 us; now 149 / 88 / 68.
 constexpr int MM_KC = 256, MM_U = 8;
 
 template <int NC>
-struct ColVec;
+struct MmVec;
 template <>
-struct ColVec<1> {
-    typedef float T;
-    static __device__ __forceinline__ float at(float v, int) { return v; }
-};
+struct MmVec<1> { typedef float T; };
 template <>
-struct ColVec<4> {
-    typedef v4f T;
-    static __device__ __forceinline__ float at(v4f v, int c) { return v[c]; }
-};
+struct MmVec<2> { typedef float T __attribute__((ext_vector_type(2))); };
+template <>
+struct MmVec<4> { typedef v4f T; };
 
-template <int MT, int NC>
-__global__ void __launch_bounds__(256) k_matmul(float *C, const float *A, const float *B, int M,
-                                                int N, int K)
+template <int MT, int NC, int RS>
+__global__ void __launch_bounds__(256) k_matmul(float *__restrict__ C, const float *__restrict__ A,
+                                                  const float *__restrict__ B, int M, int N, int K)
 {
-    typedef typename ColVec<NC>::T bvec;
-    __shared__ __align__(16) float As[MT][MM_KC];
-    const int j = (blockIdx.x * 256 + threadIdx.x) * NC;  // first column of this thread
-    const int i0 = blockIdx.y * MT;
-    const bool live = j < N;  // NC > 1 only when N % NC == 0: all NC columns exist
+    typedef typename MmVec<NC>::T bvec;
+    constexpr int TC = 256 / RS;
+    __shared__ __align__(16) float As[MT * RS][MM_KC + 4];
+    const int j = (blockIdx.x * TC + (threadIdx.x % TC)) * NC;  // first column of this thread
+    const int r0 = RS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / TC) * MT : 0;
+    const int ib = blockIdx.y * MT * RS;  // first row of the work group
+    const bool live = j < N;  // NC > 1 only when N % NC == 0
     const bvec *b = reinterpret_cast<const bvec *>(B + (live ? j : 0));
-    const size_t ldb = (size_t)N / NC;  // row stride of B in bvec units
+    const size_t ldb = (size_t)N / NC;
     float acc[MT][NC];
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int c = 0; c < NC; ++c) acc[i][c] = 0.0f;
+    auto at = [](const bvec &v, int c) -> float {
+        if constexpr (NC == 1) return v;
+        else return v[c];
+    };
+    bvec b0[MM_U], b1[MM_U];
+    auto load_b = [&](bvec(&r)[MM_U], int k) {  // k past the last whole turn: re-read row 0, unused
+        const bvec *p = b + (k + MM_U <= K ? (size_t)k * ldb : 0);
+        const size_t st = k + MM_U <= K ? ldb : 0;
+#pragma unroll
+        for (int u = 0; u < MM_U; ++u) r[u] = p[u * st];
+    };
+    if (K > 0) load_b(b0, 0);  // K = 0: B may hold nothing
     for (int k0 = 0; k0 < K; k0 += MM_KC) {
         const int kc = K - k0 < MM_KC ? K - k0 : MM_KC;
         __syncthreads();  // the previous chunk is consumed
-        for (int e = threadIdx.x; e < MT * MM_KC; e += 256) {
+        for (int e = threadIdx.x; e < MT * RS * MM_KC; e += 256) {
             const int i = e / MM_KC, k = e - i * MM_KC;
-            As[i][k] = (i0 + i < M && k < kc) ? A[(size_t)(i0 + i) * K + k0 + k] : 0.0f;
+            As[i][k] = (ib + i < M && k < kc) ? A[(size_t)(ib + i) * K + k0 + k] : 0.0f;
         }
         __syncthreads();
-        int k = 0;
-        for (; k + MM_U <= kc; k += MM_U) {
-            bvec bv[MM_U];
+        v4f a0[MT], a1[MT];
+        auto load_a = [&](v4f(&r)[MT], int k) {  // within the padded row, also past kc
 #pragma unroll
-            for (int u = 0; u < MM_U; ++u) bv[u] = b[(size_t)(k0 + k + u) * ldb];
+            for (int i = 0; i < MT; ++i) r[i] = *reinterpret_cast<const v4f *>(&As[r0 + i][k]);
+        };
+        auto mac4 = [&](const v4f(&ar)[MT], const bvec *br) {
 #pragma unroll
-            for (int u = 0; u < MM_U; ++u)
+            for (int u = 0; u < 4; ++u)
 #pragma unroll
                 for (int i = 0; i < MT; ++i)
 #pragma unroll
-                    for (int c = 0; c < NC; ++c)
-                        acc[i][c] += As[i][k + u] * ColVec<NC>::at(bv[u], c);
+                    for (int c = 0; c < NC; ++c) acc[i][c] += ar[i][u] * at(br[u], c);
+        };
+        auto turn = [&](bvec(&cur)[MM_U], bvec(&nxt)[MM_U], int k) {
+            load_b(nxt, k0 + k + MM_U);
+            load_a(a1, k + 4);
+            __builtin_amdgcn_sched_barrier(0);
+            mac4(a0, cur);
+            __builtin_amdgcn_sched_barrier(0);
+            load_a(a0, k + 8 < MM_KC ? k + 8 : 0);
+            __builtin_amdgcn_sched_barrier(0);
+            mac4(a1, cur + 4);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        load_a(a0, 0);
+        const int kw = kc - kc % MM_U;
+        int k = 0;
+        for (; k + 2 * MM_U <= kw; k += 2 * MM_U) {
+            turn(b0, b1, k);
+            turn(b1, b0, k + MM_U);
+        }
+        if (k < kw) {  // an odd turn, in the last chunk alone
+            turn(b0, b1, k);
+            k += MM_U;
         }
         for (; k < kc; ++k) {
             const bvec bk = b[(size_t)(k0 + k) * ldb];
 #pragma unroll
             for (int i = 0; i < MT; ++i)
 #pragma unroll
-                for (int c = 0; c < NC; ++c) acc[i][c] += As[i][k] * ColVec<NC>::at(bk, c);
+                for (int c = 0; c < NC; ++c) acc[i][c] += As[r0 + i][k] * at(bk, c);
         }
     }
     if (!live) return;
 #pragma unroll
     for (int i = 0; i < MT; ++i)
-        if (i0 + i < M)
+        if (ib + r0 + i < M)
 #pragma unroll
-            for (int c = 0; c < NC; ++c) C[(size_t)(i0 + i) * N + j + c] = acc[i][c];
+            for (int c = 0; c < NC; ++c) C[(size_t)(ib + r0 + i) * N + j + c] = acc[i][c];
 }
 
 // gpu.c:144-156 per row: ss is the reference's sequential fp32 sum of the
@@ -223,29 +262,38 @@ extern "C" int ornk_matmul_f32(float *C, const float *A, const float *B, int M, 
                                hipStream_t s)
 {
     if (M <= 0 || N <= 0) return hipSuccess;
-    // rows per block-row: the smallest power of two >= M, at most 16 (a
-    // register per row and column); larger M runs ceil(M/16) block-rows.
-    // Up to 4 rows a thread takes 4 columns (one 16-byte B load per step)
-    // where N allows it (N % 4 == 0 keeps every row 16-byte aligned).
-    const int mt = M > 8 ? 16 : M > 4 ? 8 : M > 2 ? 4 : M;
-    const int nc = (mt <= 4 && N % 4 == 0 && ((uintptr_t)B & 15) == 0) ? 4 : 1;
-    const dim3 grid(blocks_for(((size_t)N + nc - 1) / nc, 256), (M + mt - 1) / mt);
-#define ORN_MM(MT_, NC_) hipLaunchKernelGGL((k_matmul<MT_, NC_>), grid, dim3(256), 0, s, C, A, B, M, N, K)
-    if (nc == 4) {
-        switch (mt) {
-        case 1: ORN_MM(1, 4); break;
-        case 2: ORN_MM(2, 4); break;
-        default: ORN_MM(4, 4); break;
-        }
-    } else {
-        switch (mt) {
-        case 1: ORN_MM(1, 1); break;
-        case 2: ORN_MM(2, 1); break;
-        case 4: ORN_MM(4, 1); break;
-        case 8: ORN_MM(8, 1); break;
-        default: ORN_MM(16, 1); break;
-        }
+    const int mt = M > 4 ? 8 : M > 2 ? 4 : M, rs = M > 8 ? 2 : 1;
+    const int gy = (M + mt * rs - 1) / (mt * rs);
+    // Columns per thread: one while its waves fit the chip three to a SIMD
+    // (1024 SIMDs), two while theirs fit two to a SIMD (8-row instances take
+    // 150 to 211 registers), else four; more columns mean fewer LDS reads per
+    // product but fewer waves.  us with one / two / four columns at K = 2048:
+    // 16 rows, N = 65,536 188 / 230 / 340, 131,072 365 / 284 / 357, 248,320
+    // 583 / 538 / 441; 8 rows, N = 190,000 274 / 300 / 323, 248,320 407 / 341
+    // / 347; 1 row, N = 65,536 106 / 122 / 167, 248,320 349 / 325 / 334.
+    const size_t waves = (((size_t)N + 63) / 64) * rs * gy;
+    int nc = waves <= 3072 ? 1 : waves <= 4096 || mt <= 4 ? 2 : 4;
+    while (nc > 1 && (N % nc || ((uintptr_t)B & (4 * nc - 1)))) nc /= 2;
+    const dim3 grid(blocks_for(((size_t)N + nc - 1) / nc, 256 / rs), gy);
+#define ORN_MM(MT_, NC_, RS_) \
+    hipLaunchKernelGGL((k_matmul<MT_, NC_, RS_>), grid, dim3(256), 0, s, C, A, B, M, N, K)
+#define ORN_MM_MT(NC_)                       \
+    switch (rs == 2 ? 16 : mt) {             \
+    case 1: ORN_MM(1, NC_, 1); break;        \
+    case 2: ORN_MM(2, NC_, 1); break;        \
+    case 4: ORN_MM(4, NC_, 1); break;        \
+    case 8: ORN_MM(8, NC_, 1); break;        \
+    default: ORN_MM(8, NC_, 2); break;       \
     }
+    if (nc == 4) {
+        if (rs == 2) ORN_MM(8, 4, 2);
+        else ORN_MM(8, 4, 1);
+    } else if (nc == 2) {
+        ORN_MM_MT(2)
+    } else {
+        ORN_MM_MT(1)
+    }
+#undef ORN_MM_MT
 #undef ORN_MM
     return hipGetLastError();
 }

@@ -141,6 +141,16 @@ def test_matmul_tiled_bit_exact(om, ctx, M, N, K):
         b.free()
 
 
+@pytest.mark.parametrize("M,N,K", [(8, 196672, 9), (5, 196610, 24), (16, 98312, 17), (9, 131076, 8),
+                                   (16, 131080, 31), (12, 131074, 3), (4, 196610, 7),
+                                   (33, 65540, 264)])
+def test_matmul_column_split_bit_exact(om, ctx, M, N, K):
+    """The products with enough columns for two or four per thread, at odd
+    widths that leave fewer, with one and two turns of 8 k's and a remainder:
+    bit-identical to the sequential sums."""
+    test_matmul_tiled_bit_exact(om, ctx, M, N, K)
+
+
 @pytest.mark.parametrize("dim", [4, 64, 2048])
 def test_rmsnorm(om, ctx, dim):
     """t_gpu_metal.c:189-343 (1e-5 / 1e-4) -- here bit-exact with gpu.c:144-156."""
