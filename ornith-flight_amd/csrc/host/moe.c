@@ -1033,7 +1033,10 @@ static plan_t make_plan(const ornith_moe_shape *sh, int T, int use_mfma)
  * (D / ornk_file_down_cols() per item and slice): these kernels need
  * several rounds of work groups to hide their memory latency, and a wave
  * that covers one super-block uses every byte of its blocks while they are
- * cached. */
+ * cached.  Items of 64 rows are as many as fill the chip by themselves, and
+ * their split-K partials cost more than the extra work groups give: about
+ * 2048 there (1500 tokens: one slice for four, gate/up 330 -> 270 us, mid 38
+ * -> 16; 600 tokens: one for two, 253 -> 214 and 16 -> 8). */
 static plan_t make_plan_file(const ornith_moe_shape *sh, int T)
 {
     plan_t p;
@@ -1048,7 +1051,8 @@ static plan_t make_plan_file(const ornith_moe_shape *sh, int T)
     p.items_max = max_slots + (p.rows_max + p.tchunk - 1) / p.tchunk;
     int est = max_slots + p.rows_max / p.tchunk;
     if (est < 1) est = 1;
-    const int ng = 8192 / (est * (2 * H / 256)), nd = 8192 / (est * (D / ornk_file_down_cols()));
+    const int want = p.tchunk == 64 ? 2048 : 8192;
+    const int ng = want / (est * (2 * H / 256)), nd = want / (est * (D / ornk_file_down_cols()));
     int kg = pow2_floor(ng > 0 ? ng : 1), kd = pow2_floor(nd > 0 ? nd : 1);
     while (kg > 1 && (D / 256) % kg) kg /= 2;
     while (kd > 1 && (H / 256) % kd) kd /= 2;
