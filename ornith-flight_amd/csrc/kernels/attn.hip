@@ -146,6 +146,14 @@ __global__ __launch_bounds__(256) void k_attention(float *out, const float *Q, c
 //   out = O / L where the unshifted sum e^M L exceeds 1e-10, else O e^M
 // (attention.metal:60-62).
 // ---------------------------------------------------------------------------
+// Whether any of the operands is not finite (the same answer in every thread).
+__device__ __forceinline__ bool attn_bad(const int *bad, int ntq)
+{
+    int b = 0;
+    for (int i = threadIdx.x; i < 3 * ntq; i += blockDim.x) b |= bad[i];
+    return __syncthreads_or(b) != 0;
+}
+
 constexpr int AM_TK = 16;  // keys per tile
 
 template <int HD>
@@ -158,9 +166,11 @@ struct AttnLds {
 template <int HD>
 __global__ void __launch_bounds__(256) k_attn_mma(float *out, float *Op, float *mlp,
                                                   const float *Q, const float *K, const float *V,
-                                                  int seq, int hd, float scale, int tiles_per_split)
+                                                  int seq, int hd, float scale, int tiles_per_split,
+                                                  const int *bad, int ntq)
 {
     __shared__ __align__(16) AttnLds<HD> L;  // 79 KB at HD = 256
+    if (bad && !attn_bad(bad, ntq)) return;  // k_attn_pairs has taken it
     constexpr int NS = HD / 4, NC = HD / 16;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, c = lane & 15;
     const int q0 = blockIdx.x * 64 + 16 * wave;
@@ -308,24 +318,432 @@ __global__ void __launch_bounds__(256) k_attn_mma(float *out, float *Op, float *
     }
 }
 
-// Combines the key splits of k_attn_mma: one thread per output element.
+// Combines the key splits: one thread per four outputs (hd % 4 == 0).
 __global__ void k_attn_merge(float *out, const float *Op, const float *mlp, int seq, int hd,
                              int nsplit)
 {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)seq * hd) return;
-    const size_t row = i / hd, col = i - row * hd;
+    const int h4 = hd >> 2;
+    if (i >= (size_t)seq * h4) return;
+    const size_t row = i / h4, col = 4 * (i - row * h4);
     float M = -INFINITY;
     for (int sp = 0; sp < nsplit; ++sp) M = fmaxf(M, mlp[((size_t)sp * seq + row) * 2]);
-    float Ls = 0.0f, O = 0.0f;
+    float Ls = 0.0f;
+    v4f O = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int sp = 0; sp < nsplit; ++sp) {
         const float mi = mlp[((size_t)sp * seq + row) * 2];
         const float w = mi == -INFINITY ? 0.0f : expf(mi - M);
         Ls += mlp[((size_t)sp * seq + row) * 2 + 1] * w;
-        O += Op[((size_t)sp * seq + row) * hd + col] * w;
+        O += *reinterpret_cast<const v4f *>(Op + ((size_t)sp * seq + row) * hd + col) * w;
     }
     const float em = expf(M);
-    out[i] = em * Ls > 1e-10f ? O / Ls : O * em;
+    *reinterpret_cast<v4f *>(out + row * hd + col) = em * Ls > 1e-10f ? O / Ls : O * em;
+}
+
+// ---------------------------------------------------------------------------
+// The same attention with fp16 operand pairs (v_mfma_f32_32x32x16_f16), for
+// the sequences whose products, and not their launches, take the time.
+//
+// Every operand is x * s = hi + lo, s a power of two per row of Q and of K and
+// per column of V (|x * s| < 2^14; 2^13 for the softmax weights), hi and
+// lo each rounded to nearest, so hi + lo holds x to 2^-24 of itself; a product
+// is hi*hi + hi*lo + lo*hi, what is dropped is below 2^-24 of it, and the sums
+// are fp32: the rounding of fp32 products at 3/16 of their matrix time.  The
+// pairs are made once per call (k_attn_prep), not once per work group.
+// Operands that hold a NaN or an infinity take k_attn_mma instead, decided on
+// the device (bad[]).
+//
+// Work group: 4 waves of 32 query rows each and one split of the keys, tiles
+// of 32 keys.  Scores are formed transposed, S^T = K Q^T, so that a lane holds
+// 16 keys of one query: the row maximum and sum are in-lane but for one
+// exchange between the lane halves, and the weights are already in the B
+// layout of O^T = V^T P^T once V^T's keys are stored in that order (key
+// position 8h + e of a step of 16 is key 4h + e for e < 4, 8 + 4h + e - 4
+// beyond).  A tile of K and V (64 KB at HD = 256) goes from memory straight
+// into LDS while the one before is used, one barrier per tile.
+//
+// What bounds it: Q's pairs and O take 256 registers at HD = 256, so a SIMD
+// holds one wave, and its matrix, exponential and LDS phases follow each
+// other: the matrix cores are 31 % busy (4096 x 256: 83 us of 110 for the
+// call; with k_attn_mma 254).  Error against 64 bits there 4e-7 (fp32: 7e-7).
+// ---------------------------------------------------------------------------
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+constexpr int AS_TK = 32, AS_ROWS = 128;  // keys per tile, query rows per work group
+
+struct AttnPrep {
+    _Float16 *q;      // [rows][hi, lo][HD]
+    uint4 *kv;        // per tile [K hi][K lo] 32 x HD, [V hi][V lo] HD x 32
+    float *qinv, *kinv, *vinv;
+    int *bad;         // [tiles][Q, K, V]: the tile's values are not all finite
+};
+
+// Column maxima of V over a slice of rows: part[blockIdx.x][HD] (hd % 4 == 0).
+constexpr int AS_PARTS = 32;
+
+__global__ void __launch_bounds__(256) k_attn_colmax(float *part, const float *V, int seq, int hd,
+                                                     int HD)
+{
+    const int per = (seq + AS_PARTS - 1) / AS_PARTS;
+    const int lo = blockIdx.x * per, hi = min(seq, lo + per);
+    const int nc = HD / 4, c = 4 * (threadIdx.x % nc), rstep = 256 / nc;
+    __shared__ __align__(16) v4f red[256];
+    v4f m = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (c < hd) {
+#pragma unroll 16
+        for (int r = lo + threadIdx.x / nc; r < hi; r += rstep) {
+            const v4f v = *reinterpret_cast<const v4f *>(V + (size_t)r * hd + c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) m[e] = fmaxf(m[e], fabsf(v[e]));
+        }
+    }
+    red[threadIdx.x] = m;
+    __syncthreads();
+    if ((int)threadIdx.x >= nc) return;
+    for (int i = 1; i < rstep; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m[e] = fmaxf(m[e], red[threadIdx.x + i * nc][e]);
+    *reinterpret_cast<v4f *>(part + (size_t)blockIdx.x * HD + c) = m;
+}
+
+__device__ __forceinline__ float attn_scale(float amax)  // power of two, amax * s in [2^13, 2^14)
+{
+    if (!(amax > 0.0f) || !(amax <= 3.0e38f)) return 1.0f;
+    int e = 13 - ilogbf(amax);
+    e = e < -126 ? -126 : (e > 126 ? 126 : e);
+    return ldexpf(1.0f, e);
+}
+
+// The 16-byte chunk j of a row of K lies at position j ^ attn_kswz(row), so that
+// 16 rows' reads of one chunk cover every LDS bank.
+template <int HD>
+__device__ __forceinline__ int attn_kswz(int r)
+{
+    return HD == 64 ? (r >> 1) & 7 : r & 15;
+}
+
+template <int HD>
+__global__ void __launch_bounds__(256) k_attn_prep(AttnPrep P, const float *part, const float *Q,
+                                                   const float *K, const float *V, int seq, int hd,
+                                                   int nt)
+{
+    constexpr int W = HD / 64;  // columns per lane of a row
+    // blockIdx.y: Q, K or V of tile blockIdx.x
+    const int t = blockIdx.x, which = blockIdx.y;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    _Float16 *kt = reinterpret_cast<_Float16 *>(P.kv) + (size_t)t * 4 * AS_TK * HD;
+    bool ok = true;
+    if (which && t >= nt) {
+        // past the last tile of keys: nothing to write but the flag
+    } else if (which < 2) {
+        const float *src = which ? K : Q;
+        constexpr int NR = AS_TK / 4;  // this wave's rows
+        float x[NR][W];
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const int r = t * AS_TK + wave * NR + i;
+#pragma unroll
+            for (int j = 0; j < W; ++j) {
+                const int c = W * lane + j;
+                x[i][j] = r < seq && c < hd ? src[(size_t)r * hd + c] : 0.0f;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const int lr = wave * NR + i, r = t * AS_TK + lr;
+            float m = 0.0f;
+#pragma unroll
+            for (int j = 0; j < W; ++j) {
+                ok = ok && fabsf(x[i][j]) <= 3.4028235e38f;
+                m = fmaxf(m, fabsf(x[i][j]));
+            }
+#pragma unroll
+            for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+            const float s = attn_scale(m);
+            _Float16 *dh = which ? kt + (size_t)lr * HD : P.q + (size_t)r * 2 * HD;
+            _Float16 *dl = which ? dh + AS_TK * HD : dh + HD;
+            _Float16 hi[W], lo[W];
+#pragma unroll
+            for (int j = 0; j < W; ++j) {
+                const float v = x[i][j] * s;
+                hi[j] = (_Float16)v;
+                lo[j] = (_Float16)(v - (float)hi[j]);
+            }
+            const int o = which ? 8 * ((W * lane / 8) ^ attn_kswz<HD>(lr)) + W * lane % 8 : W * lane;
+            __builtin_memcpy(__builtin_assume_aligned(dh + o, 2 * W), hi, 2 * W);
+            __builtin_memcpy(__builtin_assume_aligned(dl + o, 2 * W), lo, 2 * W);
+            if (lane == 0) (which ? P.kinv : P.qinv)[r] = 1.0f / s;
+        }
+    } else {
+        __shared__ float vs[HD];
+        constexpr int NV = 4 * HD / 256;  // runs of 8 keys of one column per thread
+        float x[NV][8];
+#pragma unroll
+        for (int n = 0; n < NV; ++n) {
+            const int i = tid + 256 * n, c = i % HD, ch = i / HD;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int r = t * AS_TK + 16 * (ch >> 1) + 4 * (ch & 1) + (e & 3) + 8 * (e >> 2);
+                x[n][e] = r < seq && c < hd ? V[(size_t)r * hd + c] : 0.0f;
+            }
+        }
+        if (tid < HD) {
+            float m = 0.0f;
+#pragma unroll
+            for (int i = 0; i < AS_PARTS; ++i) m = fmaxf(m, part[(size_t)i * HD + tid]);
+            const float s = attn_scale(m);
+            vs[tid] = s;
+            if (t == 0) P.vinv[tid] = 1.0f / s;
+        }
+        __syncthreads();
+        _Float16 *vt = kt + 2 * AS_TK * HD;
+#pragma unroll
+        for (int n = 0; n < NV; ++n) {
+            const int i = tid + 256 * n, c = i % HD, ch = i / HD;
+            v8h hi, lo;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                ok = ok && fabsf(x[n][e]) <= 3.4028235e38f;
+                const float v = x[n][e] * vs[c];
+                hi[e] = (_Float16)v;
+                lo[e] = (_Float16)(v - (float)hi[e]);
+            }
+            // a column's four 16-byte chunks are rotated among themselves by
+            // its number, so that 16 lanes' reads cover every LDS bank
+            const int o = c * AS_TK + 8 * (ch ^ ((c >> 2) & 3));
+            *reinterpret_cast<v8h *>(vt + o) = hi;
+            *reinterpret_cast<v8h *>(vt + AS_TK * HD + o) = lo;
+        }
+    }
+    const int any = __syncthreads_or(!ok);
+    if (tid == 0) P.bad[3 * t + which] = any;
+}
+
+// 16 bytes per lane from global memory into LDS at base + 16 * lane, base the
+// same in every lane; complete after the wave's next wait for its loads.  (As
+// asm: for the builtin the compiler waits for the load before any LDS read.)
+__device__ __forceinline__ uint32_t lds_addr(const void *p)
+{
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char *)p;
+}
+__device__ __forceinline__ void lds_load16(const void *g, uint32_t base)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                 :
+                 : "s"(__builtin_amdgcn_readfirstlane(base)), "v"(g)
+                 : "memory", "m0");
+}
+
+// Keeps a value in the accumulator half of the register file, which the matrix
+// instructions read and write directly: O and Q take it all, and left to
+// itself the compiler moves O across the halves in every tile.
+template <class T>
+__device__ __forceinline__ void agpr(T &v)
+{
+    asm volatile("" : "+a"(v));
+}
+
+template <int HD>
+struct AttnSplitLds {  // one tile's image per slot
+    _Float16 k[2][2][AS_TK * HD];  // [slot][hi, lo]
+    _Float16 v[2][2][HD * AS_TK];
+    float kinv[2][AS_TK], vinv[HD];
+};
+
+template <int HD>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+    k_attn_pairs(float *out, float *Op, float *mlp, AttnPrep P, int seq, int hd, float scale,
+                 int nt, int ntq, int tiles_per_split)
+{
+    __shared__ __align__(16) AttnSplitLds<HD> L;
+    constexpr int NK = HD / 16, NJ = HD / 32, NL = HD / 32;  // NL: 16-byte words per thread of K, of V
+    if (attn_bad(P.bad, ntq)) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane & 31, h = lane >> 5;
+    const int row = blockIdx.y * AS_ROWS + 32 * wave + q;
+    const int t_lo = blockIdx.x * tiles_per_split, t_hi = min(nt, t_lo + tiles_per_split);
+
+    v8h qh[NK], ql[NK];
+    {
+        const _Float16 *qr = P.q + (size_t)row * 2 * HD + 8 * h;
+#pragma unroll
+        for (int s = 0; s < NK; ++s) {
+            qh[s] = *reinterpret_cast<const v8h *>(qr + 16 * s);
+            ql[s] = *reinterpret_cast<const v8h *>(qr + HD + 16 * s);
+        }
+#pragma unroll
+        for (int s = 0; s < NK; ++s) {
+            agpr(qh[s]);
+            agpr(ql[s]);
+        }
+    }
+    const float qs = P.qinv[row] * scale;
+
+    // K or V of one tile straight into LDS: 1 KB per wave and load.  Tiles
+    // past the split re-read its last one, unused.
+    auto load = [&](int t, int slot) {
+        const uint4 *p = P.kv + (size_t)min(t, t_hi - 1) * (16 * HD) + 64 * wave + lane;
+        const uint32_t k = lds_addr(&L.k[slot][0][0]) + 1024 * wave;
+        const uint32_t v = lds_addr(&L.v[slot][0][0]) + 1024 * wave;
+#pragma unroll
+        for (int i = 0; i < NL; ++i) lds_load16(p + 256 * i, k + 4096 * i);
+#pragma unroll
+        for (int i = 0; i < NL; ++i) lds_load16(p + 8 * HD + 256 * i, v + 4096 * i);
+    };
+    // S^T of one tile: this lane's query, keys 8 (r / 4) + 4h + r % 4
+    // (two steps' operands are read while the two before them multiply)
+    auto scores = [&](int slot) {
+        v16f s0 = {}, s1 = {};
+        v8h kb[2][2][2];
+        auto read = [&](v8h(&r)[2][2], int s2) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int off = q * HD + 8 * ((2 * (s2 + i) + h) ^ attn_kswz<HD>(q));
+                r[i][0] = *reinterpret_cast<const v8h *>(&L.k[slot][0][off]);
+                r[i][1] = *reinterpret_cast<const v8h *>(&L.k[slot][1][off]);
+            }
+        };
+        read(kb[0], 0);
+#pragma unroll
+        for (int s = 0; s < NK; s += 2) {
+            if (s + 2 < NK) read(kb[(s / 2 + 1) & 1], s + 2);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const v8h kh = kb[(s / 2) & 1][i][0], kl = kb[(s / 2) & 1][i][1];
+                s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, qh[s + i], s0, 0, 0, 0);
+                s1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, ql[s + i], s1, 0, 0, 0);
+                s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl, qh[s + i], s0, 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        return s0 + s1;
+    };
+
+    auto read_v = [&](v8h(&r)[2][2], int slot, int j) {
+        const int c = 32 * j + q;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int off = c * AS_TK + 8 * ((2 * s + h) ^ ((c >> 2) & 3));
+            r[s][0] = *reinterpret_cast<const v8h *>(&L.v[slot][0][off]);
+            r[s][1] = *reinterpret_cast<const v8h *>(&L.v[slot][1][off]);
+        }
+    };
+
+    v16f o[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        o[j] = (v16f){};
+        agpr(o[j]);
+    }
+    float m = -INFINITY, l = 0.0f;
+
+    if (tid < HD) L.vinv[tid] = P.vinv[tid];
+    float rki = P.kinv[min(t_lo + 1, t_hi - 1) * AS_TK + (tid & (AS_TK - 1))];  // of tile t + 1
+    if (tid < AS_TK) L.kinv[0][tid] = P.kinv[t_lo * AS_TK + tid];
+    load(t_lo, 0);
+    for (int t = t_lo; t < t_hi; ++t) {
+        const int cur = (t - t_lo) & 1, nxt = cur ^ 1;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) agpr(o[j]);
+        // Tile t has arrived, and every wave is past tile t - 1, whose slot
+        // takes t + 1.
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        asm volatile("" : "+v"(rki));
+        __syncthreads();
+        if (tid < AS_TK) L.kinv[nxt][tid] = rki;
+        rki = P.kinv[min(t + 2, t_hi - 1) * AS_TK + (tid & (AS_TK - 1))];
+        load(t + 1, nxt);
+        __builtin_amdgcn_sched_barrier(0);
+        const v16f sc = scores(cur);
+        v8h vb[2][2][2];
+        read_v(vb[0], cur, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        float p[16];
+        float tm = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const v4f ki = *reinterpret_cast<const v4f *>(&L.kinv[cur][8 * i + 4 * h]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float v = sc[4 * i + e] * (ki[e] * qs);
+                p[4 * i + e] = AS_TK * t + 8 * i + 4 * h + e < seq ? v : -INFINITY;
+                tm = fmaxf(tm, p[4 * i + e]);
+            }
+        }
+        tm = fmaxf(tm, __shfl_xor(tm, 32, 64));
+        // The reference m moves only when the maximum has grown past it by a
+        // factor of 4 (weights up to 4 stay): O is then left alone in most tiles.
+        const float mn = tm > m + 1.38f ? tm : m;
+        const bool none = mn == -INFINITY;  // no key of this row seen yet
+        if (__any(mn != m)) {
+            const float corr = none ? 1.0f : expf(m - mn);
+            l *= corr;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                v16f x = o[j] * corr;
+                agpr(x);
+                o[j] = x;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) agpr(o[j]);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            p[r] = none ? 0.0f : expf(p[r] - mn);
+            l += p[r];
+        }
+        m = mn;
+        v8h ph[2], pl[2];
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float v = p[8 * s + e] * 8192.0f;
+                ph[s][e] = (_Float16)v;
+                pl[s][e] = (_Float16)(v - (float)ph[s][e]);
+            }
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            if (j + 1 < NJ) read_v(vb[(j + 1) & 1], cur, j + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const v8h vh = vb[j & 1][s][0], vl = vb[j & 1][s][1];
+                o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, ph[s], o[j], 0, 0, 0);
+                o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, pl[s], o[j], 0, 0, 0);
+                o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl, ph[s], o[j], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    l += __shfl_xor(l, 32, 64);
+    if (row >= seq) return;
+    const int nsplit = gridDim.x;
+    float f = 1.0f / 8192.0f;
+    float *po;
+    if (nsplit == 1) {
+        const float em = expf(m);
+        f *= em * l > 1e-10f ? 1.0f / l : em;
+        po = out + (size_t)row * hd;
+    } else {
+        po = Op + ((size_t)blockIdx.x * seq + row) * hd;
+        if (h == 0) {
+            mlp[((size_t)blockIdx.x * seq + row) * 2] = m;
+            mlp[((size_t)blockIdx.x * seq + row) * 2 + 1] = l;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int c = 32 * j + 8 * i + 4 * h;
+            if (c >= hd) continue;  // hd % 4 == 0
+            const v4f vi = *reinterpret_cast<const v4f *>(&L.vinv[c]);
+            v4f r;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) r[e] = o[j][4 * i + e] * f * vi[e];
+            *reinterpret_cast<v4f *>(po + c) = r;
+        }
 }
 
 // attention.metal:80-108: thread i updates column i of the dim x dim state,
@@ -397,10 +815,98 @@ static int attn_splits(int seq)
     return ns > nt ? nt : ns;
 }
 
+static int attn_hd(int hd) { return hd <= 64 ? 64 : hd <= 128 ? 128 : 256; }
+
+// Pairs (k_attn_pairs) from where their three more launches are paid back;
+// fp32 / pairs, us per call: hd = 256 1400 keys 67 / 65, 1700 77 / 66, 4096
+// 254 / 110; hd = 128 1400 54 / 57, 1700 58 / 57, 4096 154 / 82; hd = 64 1700
+// 44 / 48, 2048 49 / 50, 3000 70 / 58.
+static int attn_pairs(int seq, int hd)
+{
+    const int HD = attn_hd(hd);
+    return seq >= (HD == 256 ? 1536 : HD == 128 ? 1700 : 2176);
+}
+
+static int attn_pair_splits(int seq, int *per)
+{
+    const int nq = (seq + AS_ROWS - 1) / AS_ROWS, nt = (seq + AS_TK - 1) / AS_TK;
+    int ns = 256 / nq;
+    ns = ns < 1 ? 1 : ns > nt ? nt : ns;
+    *per = (nt + ns - 1) / ns;
+    return (nt + *per - 1) / *per;  // every split holds at least one tile
+}
+
+struct AttnWs {
+    size_t q, kv, qinv, kinv, vinv, bad, part, op, ml, bytes;
+};
+
+static AttnWs attn_ws(int seq, int hd)
+{
+    const int HD = attn_hd(hd), rq = (seq + AS_ROWS - 1) / AS_ROWS * AS_ROWS;
+    const int rk = (seq + AS_TK - 1) / AS_TK * AS_TK;
+    int per;
+    const int ns = attn_pair_splits(seq, &per);
+    AttnWs w;
+    size_t off = 0;
+    auto take = [&](size_t n) {
+        const size_t o = off;
+        off += (n + 255) & ~(size_t)255;
+        return o;
+    };
+    w.q = take((size_t)rq * HD * 4);
+    w.kv = take((size_t)rk * HD * 8);
+    w.qinv = take((size_t)rq * 4);
+    w.kinv = take((size_t)rk * 4);
+    w.vinv = take((size_t)HD * 4);
+    w.bad = take((size_t)(rq / AS_TK) * 12);
+    w.part = take((size_t)AS_PARTS * HD * 4);
+    w.op = take(ns > 1 ? (size_t)ns * seq * hd * 4 : 0);
+    w.ml = take(ns > 1 ? (size_t)ns * seq * 8 : 0);
+    w.bytes = off;
+    return w;
+}
+
 extern "C" size_t ornk_attention_mma_ws(int seq, int hd)
 {
+    if (attn_pairs(seq, hd)) return attn_ws(seq, hd).bytes;
     const int ns = attn_splits(seq);
     return ns > 1 ? (size_t)ns * seq * (hd + 2) * sizeof(float) : 0;
+}
+
+static void attn_merge(float *out, const float *Op, const float *mlp, int seq, int hd, int ns,
+                       hipStream_t s)
+{
+    const size_t n = (size_t)seq * (hd / 4);
+    hipLaunchKernelGGL(k_attn_merge, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, out, Op,
+                       mlp, seq, hd, ns);
+}
+
+template <int HD>
+static void attn_pairs_launch(float *out, const float *Q, const float *K, const float *V, int seq,
+                              int hd, float scale, uint8_t *ws, hipStream_t s)
+{
+    const AttnWs w = attn_ws(seq, hd);
+    const int nq = (seq + AS_ROWS - 1) / AS_ROWS, nt = (seq + AS_TK - 1) / AS_TK;
+    const int ntq = nq * (AS_ROWS / AS_TK);
+    int per;
+    const int ns = attn_pair_splits(seq, &per);
+    AttnPrep P;
+    P.q = reinterpret_cast<_Float16 *>(ws + w.q);
+    P.kv = reinterpret_cast<uint4 *>(ws + w.kv);
+    P.qinv = reinterpret_cast<float *>(ws + w.qinv);
+    P.kinv = reinterpret_cast<float *>(ws + w.kinv);
+    P.vinv = reinterpret_cast<float *>(ws + w.vinv);
+    P.bad = reinterpret_cast<int *>(ws + w.bad);
+    float *part = reinterpret_cast<float *>(ws + w.part);
+    float *Op = reinterpret_cast<float *>(ws + w.op), *mlp = reinterpret_cast<float *>(ws + w.ml);
+    hipLaunchKernelGGL(k_attn_colmax, dim3(AS_PARTS), dim3(256), 0, s, part, V, seq, hd, HD);
+    hipLaunchKernelGGL(k_attn_prep<HD>, dim3(ntq, 3), dim3(256), 0, s, P, part, Q, K, V, seq, hd, nt);
+    hipLaunchKernelGGL(k_attn_pairs<HD>, dim3(ns, nq), dim3(256), 0, s, out, Op, mlp, P, seq, hd,
+                       scale, nt, ntq, per);
+    // the same splits (twice as many tiles of half the keys), the same partials
+    hipLaunchKernelGGL(k_attn_mma<HD>, dim3((seq + 63) / 64, ns), dim3(256), 0, s, out, Op, mlp, Q, K,
+                       V, seq, hd, scale, per * (AS_TK / AM_TK), P.bad, ntq);
+    if (ns > 1) attn_merge(out, Op, mlp, seq, hd, ns, s);
 }
 
 extern "C" int ornk_attention_mma(float *out, const float *Q, const float *K, const float *V,
@@ -408,6 +914,14 @@ extern "C" int ornk_attention_mma(float *out, const float *Q, const float *K, co
 {
     if (seq <= 0 || hd <= 0) return hipSuccess;
     if (hd % 4 || hd > 256) return hipErrorInvalidValue;
+    if (attn_pairs(seq, hd)) {
+        if (!ws) return hipErrorInvalidValue;
+        uint8_t *w = static_cast<uint8_t *>(ws);
+        if (hd <= 64) attn_pairs_launch<64>(out, Q, K, V, seq, hd, scale, w, s);
+        else if (hd <= 128) attn_pairs_launch<128>(out, Q, K, V, seq, hd, scale, w, s);
+        else attn_pairs_launch<256>(out, Q, K, V, seq, hd, scale, w, s);
+        return hipGetLastError();
+    }
     const int nt = (seq + AM_TK - 1) / AM_TK;
     int ns = attn_splits(seq);
     const int per = (nt + ns - 1) / ns;
@@ -418,16 +932,12 @@ extern "C" int ornk_attention_mma(float *out, const float *Q, const float *K, co
     const dim3 grid((seq + 63) / 64, ns);
 #define ORN_ATT(HD_)                                                                          \
     hipLaunchKernelGGL(k_attn_mma<HD_>, grid, dim3(256), 0, s, out, Op, mlp,                  \
-                       Q, K, V, seq, hd, scale, per)
+                       Q, K, V, seq, hd, scale, per, (const int *)nullptr, 0)
     if (hd <= 64) ORN_ATT(64);
     else if (hd <= 128) ORN_ATT(128);
     else ORN_ATT(256);
 #undef ORN_ATT
-    if (ns > 1) {
-        const size_t n = (size_t)seq * hd;
-        hipLaunchKernelGGL(k_attn_merge, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, out,
-                           Op, mlp, seq, hd, ns);
-    }
+    if (ns > 1) attn_merge(out, Op, mlp, seq, hd, ns, s);
     return hipGetLastError();
 }
 

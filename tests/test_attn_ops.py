@@ -157,6 +157,72 @@ def test_gpu_attention(om, ctx, seq, hd):
         b.free()
 
 
+def run_attention(om, ctx, Q, K, V, in_place=False):
+    bufs = [ctx.upload(a) for a in (Q, K, V)]
+    ob = bufs[0] if in_place else ctx.alloc(Q.nbytes)
+    om.lib().gpu_attention(ctx.ptr, ob.ptr, bufs[0].ptr, bufs[1].ptr, bufs[2].ptr, *Q.shape)
+    got = ctx.download(ob, np.float32, Q.shape)
+    for b in set(bufs + [ob]):
+        b.free()
+    return got
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("seq,hd", [(1536, 256), (1541, 252), (1700, 128), (1763, 96), (2176, 64),
+                                    (2209, 60), (4129, 256)])
+def test_gpu_attention_pairs(om, ctx, seq, hd):
+    """Sequences long enough for the fp16-pair kernel, at and past its tiles
+    of 32 keys and 128 rows and its padded head dims.  Columns of V, rows of
+    Q and of K have scales far apart (a power of two each, taken out of the
+    other operand, so that the scores stay the plain ones'): within 2e-6 of
+    fp64 in every column by itself.  Also with out = Q."""
+    rng = np.random.default_rng(seq + hd)
+    Q, K, V = (f32(rng.standard_normal((seq, hd))) for _ in range(3))
+    u = f32(2.0 ** rng.integers(-6, 7, hd))
+    Q, K = Q * u, K / u
+    V = V * f32(2.0 ** rng.integers(-40, 41, hd))
+    ref = attention64(Q, K, V)
+    got = run_attention(om, ctx, Q, K, V)
+    err = (np.abs(got - ref).max(axis=0) / np.abs(ref).max(axis=0)).max()
+    assert err < 2e-6, err
+    assert np.array_equal(run_attention(om, ctx, Q, K, V, in_place=True), got)
+
+
+@pytest.mark.gpu
+def test_gpu_attention_pairs_growing_and_large_scores(om, ctx):
+    """Keys ordered by their score, so that the running maximum grows in
+    every tile, and scores of a few hundred (as in the test below, whose
+    tolerance they have)."""
+    rng = np.random.default_rng(3)
+    seq, hd = 2200, 64
+    Q, K, V = (f32(rng.standard_normal((seq, hd))) for _ in range(3))
+    Q = np.repeat(Q[:1], seq, axis=0) * f32(rng.uniform(0.5, 2.0, (seq, 1)))
+    K = K[np.argsort(K @ Q[0])]
+    ref = attention64(Q, K, V)
+    assert np.abs(run_attention(om, ctx, Q, K, V) - ref).max() < 2e-6 * np.abs(ref).max()
+    got = run_attention(om, ctx, Q * 6, K * 6, V)
+    assert np.allclose(got, attention64(Q * 6, K * 6, V), rtol=1e-4, atol=5e-5)
+
+
+@pytest.mark.gpu
+def test_gpu_attention_pairs_not_finite(om, ctx):
+    """An infinity or NaN stays where fp32 arithmetic puts it: the pair
+    kernel leaves such operands to the fp32 one."""
+    rng = np.random.default_rng(4)
+    seq, hd = 2180, 64
+    Q, K, V = (f32(rng.standard_normal((seq, hd))) for _ in range(3))
+    ref = attention64(Q, K, V)
+    V[2179, 3] = np.inf
+    V[0, 63] = np.nan
+    got = run_attention(om, ctx, Q, K, V)
+    cols = (np.arange(hd) != 3) & (np.arange(hd) != 63)
+    assert (got[:, 3] == np.inf).all() and np.isnan(got[:, 63]).all()
+    err = np.abs(got - ref)[:, cols].max() / np.abs(ref).max()
+    assert err < 2e-6, err
+    K[100, 0] = np.nan
+    assert np.isnan(run_attention(om, ctx, Q, K, V)).all()
+
+
 @pytest.mark.gpu
 def test_gpu_attention_large_scores(om, ctx):
     """Scores above 88: the shader's unshifted e^s overflows (the oracle
