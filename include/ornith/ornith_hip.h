@@ -193,7 +193,8 @@ typedef struct {
     int has_shared; /* 1: one always-on shared expert (model.c:1001-1007) */
     int prefill_layout; /* 1: also keep the MFMA layouts of every expert (about
                            1.13x the quantized bytes more) beside the GGUF
-                           blocks; 0: GGUF blocks only (VALU path); 2: the MFMA
+                           blocks; 0: GGUF blocks only (MFMA kernels that
+                           read the blocks); 2: the MFMA
                            layouts only: blocks are packed as they are uploaded
                            or generated and not kept (1.13x the GGUF bytes in
                            all); gpu_moe_store_get_experts, the VALU path and
@@ -317,15 +318,15 @@ int gpu_moe_store_cache_stats(gpu_context *ctx, ornith_moe_store *store,
 enum { ORN_ROUTE_RENORM = 0, ORN_ROUTE_LITERAL = 1 };
 #define ORN_MOE_ASYNC 1u /* return without synchronising the stream */
 #define ORN_MOE_NORM 2u  /* expert input = rmsnorm(x, layer norm weights) */
-/* Expert-product kernels.  Default: the MFMA kernels (prefill layout, fp16
- * hi+lo activations, fp32 accumulate; decode-shaped instances up to 64
- * tokens, grouped GEMMs above) when the batch has at least
- * ORN_MOE_MFMA_MIN_TOKENS tokens and the store keeps the prefill layouts
- * (Q6_K sub-block scales of any magnitude: above 64 the down kernels split
- * sc * q in two exact fp16 operands); else the VALU matvec kernels (fp32
+/* Expert-product kernels.  Default: the MFMA kernels (fp16 hi+lo activations,
+ * fp32 accumulate; Q6_K sub-block scales of any magnitude: above 64 the down
+ * kernels split sc * q in two exact fp16 operands).  With the prefill layouts
+ * they are decode-shaped instances for small and thinly spread batches and
+ * grouped GEMMs above; a store of GGUF blocks alone has its own, which read
+ * the blocks.  ORN_MOE_PATH_VALU selects the VALU matvec kernels (fp32
  * throughout). */
 #define ORN_MOE_PATH_VALU 4u /* force the VALU kernels */
-#define ORN_MOE_PATH_MFMA 8u /* force the MFMA kernels (EUNSUPPORTED if unavailable) */
+#define ORN_MOE_PATH_MFMA 8u /* force the prefill layouts' MFMA kernels (EUNSUPPORTED without) */
 #define ORN_MOE_MFMA_MIN_TOKENS 1
 /* Replay as a HIP graph: the first call with a given (layer(s), token
  * count, route mode, flags, buffer addresses) runs normally and records its

@@ -937,6 +937,7 @@ int gpu_moe_store_get_experts(gpu_context *ctx, ornith_moe_store *st, int layer,
 typedef struct {
     int ks_gu, ks_dn, rows_max, items_max, tchunk;
     int use_dec; /* MFMA path with the decode-shaped kernels (items <= 16 rows) */
+    int use_blk; /* MFMA kernels on vec@mat blocks (items <= 32 rows) */
 } plan_t;
 
 static int pow2_floor(int v)
@@ -954,7 +955,7 @@ static int pow2_floor(int v)
 static plan_t make_plan(const ornith_moe_shape *sh, int T, int use_mfma)
 {
     plan_t p;
-    p.use_dec = 0;
+    memset(&p, 0, sizeof p);
     const int k = sh->top_k, E = sh->n_experts;
     const int D = sh->d_model, H = sh->hidden;
     /* MFMA work items hold at most one 16-row tile (the decode kernels) at
@@ -1061,6 +1062,33 @@ static plan_t make_plan_file(const ornith_moe_shape *sh, int T)
     return p;
 }
 
+/* MFMA kernels on vec@mat blocks: items of <= 16 rows up to 64 tokens, <= 32
+ * above; the reduction is split so that gate/up and down have about 4096 work
+ * groups of two waves (four rounds of the chip at their occupancy) but keep
+ * slices of at least 4 steps.  0 if the shape's slices are not taken. */
+static int make_plan_blk(const ornith_moe_shape *sh, int T, plan_t *out)
+{
+    plan_t p;
+    memset(&p, 0, sizeof p);
+    const int k = sh->top_k, E = sh->n_experts, D = sh->d_model, H = sh->hidden;
+    p.use_blk = 1;
+    p.tchunk = T <= 64 ? 16 : 32;
+    p.rows_max = T * k + (sh->has_shared ? T : 0);
+    const int max_slots = (T * k < E ? T * k : E) + (sh->has_shared ? 1 : 0);
+    p.items_max = max_slots + (p.rows_max + p.tchunk - 1) / p.tchunk;
+    const int est = max_slots + p.rows_max / p.tchunk;
+    const int ng = 4096 / (est * (2 * H / 256)), nd = 4096 / (est * (D / 256));
+    int kg = pow2_floor(ng > 0 ? ng : 1), kd = pow2_floor(nd > 0 ? nd : 1);
+    while (D / 32 / kg > 64) kg *= 2;
+    while (kg > 1 && ((D / 32) % kg || D / 32 / kg < 4)) kg /= 2;
+    while (kd > 1 && ((H / 32) % kd || H / 32 / kd < 4 || kd > 16)) kd /= 2;
+    p.ks_gu = kg;
+    p.ks_dn = kd;
+    if (!ornk_blk_supported(D / 32 / kg, H / 32 / kd)) return 0;
+    *out = p;
+    return 1;
+}
+
 static int check_buf(const gpu_buffer *b, size_t bytes) { return b && b->size >= bytes; }
 
 static int launch(gpu_context *ctx, const char *name, int (*fn)(const ornk_moe_args *, hipStream_t),
@@ -1134,7 +1162,11 @@ static int moe_forward_dev(gpu_context *ctx, ornith_moe_store *st, int layer, co
         use_mfma = 1;
     }
     if (file) use_mfma = 0;  /* the mid and combine steps run as on the VALU path */
-    plan_t p = file ? make_plan_file(sh, T) : make_plan(sh, T, use_mfma);
+    plan_t p;
+    /* A store of blocks alone: the MFMA kernels that read them, unless the
+     * call forces the VALU kernels. */
+    const int blk = !file && !mfma_ok && !(flags & ORN_MOE_PATH_VALU) && make_plan_blk(sh, T, &p);
+    if (!blk) p = file ? make_plan_file(sh, T) : make_plan(sh, T, use_mfma);
 
     /* Certified routing of the smallest decode batches (router_cert.hip):
      * logits, top-k and dispatch in one launch.  Streamed stores keep it too
@@ -1168,8 +1200,8 @@ static int moe_forward_dev(gpu_context *ctx, ornith_moe_store *st, int layer, co
     CARVE(o_gu, (size_t)p.ks_gu * p.rows_max * 2 * H * 4);
     CARVE(o_mid, (size_t)p.rows_max * H * 4);
     CARVE(o_dn, (size_t)p.ks_dn * p.rows_max * D * 4);
-    CARVE(o_xamax, use_mfma ? (size_t)T * 4 : 0);
-    CARVE(o_midamax, use_mfma ? (size_t)p.rows_max * 4 : 0);
+    CARVE(o_xamax, use_mfma || blk ? (size_t)T * 4 : 0);
+    CARVE(o_midamax, use_mfma || blk ? (size_t)p.rows_max * 4 : 0);
     CARVE(o_fxh, file ? (size_t)T * D * 2 : 0);
     CARVE(o_fxl, file ? (size_t)T * D * 2 : 0);
     CARVE(o_fsh, file ? (size_t)T * (D / 32) * 2 : 0);
@@ -1246,7 +1278,7 @@ static int moe_forward_dev(gpu_context *ctx, ornith_moe_store *st, int layer, co
     a.gu_part = (float *)(ws + o_gu);
     a.mid = (float *)(ws + o_mid);
     a.dn_part = (float *)(ws + o_dn);
-    a.use_mfma = use_mfma;
+    a.use_mfma = use_mfma || blk;
     a.q6_wide = st->q6_scmax && st->q6_scmax[layer] > 64; /* held by MFMA-layout stores */
     if (use_mfma && !st->cache) {  /* a streamed store's slot arrays come from the cache */
         const size_t slot0 = (size_t)layer * E1, DH = (size_t)D * H;
@@ -1263,7 +1295,7 @@ static int moe_forward_dev(gpu_context *ctx, ornith_moe_store *st, int layer, co
         a.dn_pf.dd = (const float *)((const uint8_t *)st->dd + slot0 * (DH / 64));
         a.dn_pf.dmax = st->dmax + slot0 * 3;
     }
-    if (use_mfma) {
+    if (use_mfma || blk) {
         a.x_amax = (float *)(ws + o_xamax);
         a.router_amax = 1;  /* every routing kernel writes the rows' max |x| */
         a.mid_amax = (float *)(ws + o_midamax);
@@ -1316,6 +1348,8 @@ static int moe_forward_dev(gpu_context *ctx, ornith_moe_store *st, int layer, co
     }
     if (p.use_dec) {
         if ((rc = launch_k(ctx, "moe_gateup_dec", ornk_moe_gateup_dec, &a))) return rc;
+    } else if (p.use_blk) {
+        if ((rc = launch_k(ctx, "moe_gateup_blk", ornk_moe_gateup_blk, &a))) return rc;
     } else if (use_mfma) {
         if ((rc = launch_k(ctx, "moe_gateup_mfma", ornk_moe_gateup_mfma, &a))) return rc;
     } else {
@@ -1328,6 +1362,8 @@ static int moe_forward_dev(gpu_context *ctx, ornith_moe_store *st, int layer, co
     if (!fused_mid && (rc = launch_k(ctx, "moe_mid", ornk_moe_mid, &a))) return rc;
     if (p.use_dec) {
         if ((rc = launch_k(ctx, "moe_down_dec", ornk_moe_down_dec, &a))) return rc;
+    } else if (p.use_blk) {
+        if ((rc = launch_k(ctx, "moe_down_blk", ornk_moe_down_blk, &a))) return rc;
     } else if (use_mfma) {
         if ((rc = launch_k(ctx, "moe_down_mfma", ornk_moe_down_mfma, &a))) return rc;
     } else {

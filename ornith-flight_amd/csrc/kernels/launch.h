@@ -199,7 +199,7 @@ typedef struct {
     float *gu_part;   /* [ks_gu][rows_max][2H] */
     float *mid;       /* [rows_max][H] */
     float *dn_part;   /* [ks_dn][rows_max][D] */
-    /* MFMA path (ks_gu = ks_dn = 1, tchunk <= 64) */
+    /* MFMA paths (tchunk <= 64): the mid step writes mid_amax */
     int use_mfma;
     ornk_gu_prefill gu_pf;
     ornk_dn_prefill dn_pf;
@@ -255,6 +255,11 @@ int ornk_moe_gateup_dec(const ornk_moe_args *a, hipStream_t s);
 /* 1 if the decode instances cover kt_gu (D/32/ks_gu) and kt_dn (H/32/ks_dn). */
 int ornk_dec_supported(int kt_gu, int kt_dn);
 int ornk_moe_down_dec(const ornk_moe_args *a, hipStream_t s);
+/* The same from vec@mat blocks (items of <= 32 rows): 1 if slices of kt_gu =
+ * D/32/ks_gu and kt_dn = H/32/ks_dn steps are taken. */
+int ornk_blk_supported(int kt_gu, int kt_dn);
+int ornk_moe_gateup_blk(const ornk_moe_args *a, hipStream_t s);
+int ornk_moe_down_blk(const ornk_moe_args *a, hipStream_t s);
 /* out[r] = max_k |x[r][k]| (D a multiple of 4). */
 int ornk_file_supported(int D, int H);
 /* Output columns of one work group of the file-orientation down kernel. */

@@ -1,0 +1,105 @@
+"""A store of vec@mat blocks alone (prefill_layout = 0) on the matrix-core
+kernels that read the blocks: every forward against the oracle (indices
+exact, outputs <= 1e-5 of the row's largest, the bar of the other expert
+paths) and against the same call forced onto the fp32 kernels.
+"""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx(om):
+    c = om.Context()
+    yield c
+    c.close()
+
+
+@pytest.fixture(scope="module")
+def om():
+    import ornith_moe
+    return ornith_moe
+
+
+def wide_scales(om, syn, seed):
+    """Q6_K sub-scales over the int8 range, each block's first at an end."""
+    rng = np.random.default_rng(seed)
+    b = syn.down.reshape(-1, om.Q6K_BYTES)
+    sc = rng.integers(-128, 128, (b.shape[0], 16))
+    sc[:, 0] = np.where(rng.random(b.shape[0]) < 0.5, -128, 127)
+    b[:, 192:208] = sc.astype(np.int8).view(np.uint8)
+
+
+def forward(om, ctx, st, x, flags, mode=0, names=None):
+    T, D = x.shape
+    xb, ob = ctx.upload(x), ctx.alloc(x.nbytes)
+    ib, wb = ctx.alloc(T * st.k * 4), ctx.alloc(T * st.k * 4)
+    if names is not None:
+        om.lib().gpu_profile_enable(ctx.ptr, 1)
+        om.lib().gpu_profile_reset(ctx.ptr)
+    st.forward(0, xb, T, ob, resid=xb, idx=ib, w=wb, flags=flags, mode=mode)
+    if names is not None:
+        names += [n for n, (_, calls) in om.profile(ctx).items() if calls]
+        om.lib().gpu_profile_enable(ctx.ptr, 0)
+    got = (ctx.download(ob, np.float32, x.shape), ctx.download(ib, np.uint32, (T, st.k)),
+           ctx.download(wb, np.float32, (T, st.k)))
+    for b in (xb, ob, ib, wb):
+        b.free()
+    return got
+
+
+def row_err(a, ref):
+    return (np.abs(a - ref).max(axis=1) / np.abs(ref).max(axis=1)).max()
+
+
+# Shapes: one block column and several, slices from 4 steps to the longest
+# taken (2048 / 32 = 64); token counts at one and two row tiles' edges, the
+# step from 16- to 32-row items (64 / 65), experts over several items.
+@pytest.mark.parametrize("D,H,E,k,wide,shared", [(256, 256, 4, 2, False, True),
+                                                 (512, 1024, 6, 3, True, True),
+                                                 (2048, 256, 3, 2, True, False),
+                                                 (2048, 512, 16, 8, True, True)])
+@pytest.mark.parametrize("T", [1, 15, 17, 64, 65, 131])
+def test_blocks_mfma(om, ctx, D, H, E, k, wide, shared, T):
+    syn = om.SyntheticLayer(7 * D + H, 0, D, H, E, shared)
+    if wide:
+        wide_scales(om, syn, H)
+    st = om.Store(ctx, 1, D, H, E, k, shared, prefill_layout=False)
+    st.load_layer(0, syn)
+    x = om.synth_normal(T, om.synth_stream(0, om.SYN_ACT, 0), T * D, 1.0).reshape(T, D)
+    x[T // 2] *= 1e4  # rows of very different size in one item
+    names = []
+    out, idx, w = forward(om, ctx, st, x, om.MOE_NORM if T % 2 else 0, names=names)
+    assert {"moe_gateup_blk", "moe_down_blk"} <= set(names)
+    valu, vidx, _ = forward(om, ctx, st, x, (om.MOE_NORM if T % 2 else 0) | om.MOE_PATH_VALU)
+    kw = {"sh_" + n: syn.shared(n) for n in ("gate", "up", "down")} if shared else {}
+    ref, ridx, rw = O.moe_layer(D=D, H=H, E=E, k=k, x=x, resid=x, router_W=syn.router,
+                                norm_w=np.ones(D, np.float32) if T % 2 else None,
+                                gate=syn.routed("gate"), up=syn.routed("up"),
+                                down=syn.routed("down"), **kw)
+    assert np.array_equal(idx, ridx) and np.array_equal(vidx, ridx)
+    assert np.allclose(w, rw, rtol=1e-5)
+    assert row_err(out, ref) <= 1e-5 and row_err(valu, ref) <= 1e-5
+    st.close()
+
+
+def test_blocks_mfma_row_isolation(om, ctx):
+    """A NaN row poisons its own output and no other, and an expert's rows may
+    come in any order."""
+    D, H, E, k, T = 256, 256, 4, 2, 40
+    syn = om.SyntheticLayer(3, 0, D, H, E, True)
+    st = om.Store(ctx, 1, D, H, E, k, True, prefill_layout=False)
+    st.load_layer(0, syn)
+    x = om.synth_normal(5, om.synth_stream(0, om.SYN_ACT, 0), T * D, 1.0).reshape(T, D)
+    out, idx, _ = forward(om, ctx, st, x, 0)
+    y = x.copy()
+    y[11, 3] = np.nan
+    got, _, _ = forward(om, ctx, st, y, 0)
+    keep = np.arange(T) != 11
+    assert np.isnan(got[11]).all() and np.array_equal(got[keep], out[keep])
+    perm = np.random.default_rng(1).permutation(T)
+    assert np.array_equal(forward(om, ctx, st, x[perm], 0)[0], out[perm])
+    st.close()
