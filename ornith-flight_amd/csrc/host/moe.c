@@ -960,12 +960,15 @@ static plan_t make_plan(const ornith_moe_shape *sh, int T, int use_mfma)
     const int D = sh->d_model, H = sh->hidden;
     /* MFMA work items hold at most one 16-row tile (the decode kernels) at
      * decode sizes, two (the decode kernels' two-tile instances) above 64
-     * tokens wherever the batch averages at most 16 rows per expert, four
-     * (the prefill grouped GEMMs) beyond.  Skewed batches of the middle
-     * kind (a few hot experts, many cold ones) then split each hot expert
-     * into items of 32 rows instead of running every cold expert through a
-     * 64-row tile: an item costs its weight conversion whatever its rows. */
-    p.tchunk = use_mfma ? (T <= 64 ? 16 : T * k <= 16 * E ? 32 : 64) : (T <= 64 ? 2 : 8);
+     * tokens wherever the batch averages at most 32 rows per expert, four
+     * (the prefill grouped GEMMs) beyond: with 256 experts and top 8 the
+     * layer takes 288 / 324 us (two tiles / four) at 600 tokens, 340 / 362
+     * at 900, 369 / 381 at 1024, 389 / 391 at 1100, 497 / 425 at 1400.
+     * Skewed batches (a few hot experts, many cold ones) then split each
+     * hot expert into items of 32 rows instead of running every cold expert
+     * through a 64-row tile: an item costs its weight conversion whatever
+     * its rows. */
+    p.tchunk = use_mfma ? (T <= 64 ? 16 : T * k <= 32 * E ? 32 : 64) : (T <= 64 ? 2 : 8);
     p.rows_max = T * k + (sh->has_shared ? T : 0);
     const int max_slots = (T * k < E ? T * k : E) + (sh->has_shared ? 1 : 0);
     p.items_max = max_slots + (p.rows_max + p.tchunk - 1) / p.tchunk;
@@ -1010,7 +1013,13 @@ static plan_t make_plan(const ornith_moe_shape *sh, int T, int use_mfma)
             int dg = pow2_floor(ng > 0 ? ng : 1);
             while (dg > 1 && (D / 32) % dg) dg /= 2;
             while (dg > 1 && D / 32 / dg < 4) dg /= 2;
-            while ((D / 32) % (2 * dg) == 0 && D / 32 / dg > 16) dg *= 2;
+            /* slices of 32 steps once two-tile items are many enough to fill
+             * the chip with half as many work groups: the mid step then reads
+             * half the partials (512 tokens gate/up 111 -> 105 us, mid 15 ->
+             * 10; 709: 124 -> 114 and 20 -> 13; 128 tokens of a skewed batch
+             * 34.0 -> 35.1 and 5.1 -> 4.4) */
+            const int most = p.tchunk == 32 && T >= 192 ? 32 : 16;
+            while ((D / 32) % (2 * dg) == 0 && D / 32 / dg > most) dg *= 2;
             int dd = 1;
             while ((H / 32) % (2 * dd) == 0 && H / 32 / dd > 8) dd *= 2;
             /* Two-tile items (32 rows): down unsplit when a slice of all H
