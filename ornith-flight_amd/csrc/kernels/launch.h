@@ -225,7 +225,9 @@ int ornk_moe_norm(const ornk_moe_args *a, hipStream_t s);
 int ornk_moe_route(const ornk_moe_args *a, hipStream_t s);
 /* Batches the one-wave-per-(token, 8 experts) router takes (and that can
  * produce x_amax on the side). */
-#define ORN_ROUTER_PC_MAX_T 64
+/* (Beyond, a separate norm and the staged router: with the norm 155 us for the
+ * layer at 40 tokens either way, 191 -> 177 at 64.) */
+#define ORN_ROUTER_PC_MAX_T 40
 int ornk_router_pc_supported(int T, int D);
 /* Whether the decode down kernel forms mid itself (the mid step is then
  * skipped): one token, 16 gate/up split-K slices, 8-step down slices. */

@@ -8,7 +8,7 @@
 //
 // The MoE path computes every logit with exactly that arithmetic, one chain
 // per (token, expert), all chains in parallel (k_router_pc for decode-sized
-// batches, k_router_dec / k_router_seq above), so the logits are
+// batches, k_router_seq above), so the logits are
 // bit-identical to the reference's by construction.  Top-k selection and
 // the dispatch that follows it: dispatch.hip.
 #include "common.h"
@@ -17,6 +17,8 @@
 
 #include <float.h>
 #include <limits.h>
+
+#include <utility>
 
 
 namespace {
@@ -142,12 +144,25 @@ __device__ void exact_select(float val, int n, int k, float *vals_s, int *idx_s,
 // ORN_RPF chunks in flight in registers, copies chunk c into one of two LDS
 // slots, and every chain then consumes the chunk in d order.
 // ---------------------------------------------------------------------------
+// Lane N of every row of 16 lanes, in all lanes of the row.
+template <int N>
+__device__ __forceinline__ float row_bcast(float v)
+{
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x150 + N, 0xF, 0xF, true));
+}
+
+template <class F, int... G>
+__device__ __forceinline__ void for_each_quad(F f, std::integer_sequence<int, G...>)
+{
+    (f(std::integral_constant<int, G>{}), ...);
+}
+
 #define ORN_RDC 64                 // d values per chunk (half the barriers of 32:
                                    // 76.0 -> 72.8 us at 2048 tokens)
 #define ORN_RPF 4                  // chunks in flight
 #define ORN_RWS4 (ORN_RDC / 4 + 1) // LDS row stride of a weight row, in float4 (padded)
 
-template <int TPW>
+template <int TPW, int NB>
 __global__ void __launch_bounds__(256)
     k_router_seq(const float *__restrict__ x, const float *__restrict__ Wq,
                  const float *__restrict__ bias, int T, int D, int E,
@@ -237,42 +252,35 @@ __global__ void __launch_bounds__(256)
                 __syncthreads();
                 const v4f *wr = &wl[sl][lane * ORN_RWS4];
                 const v4f *xr = &xl[sl][wave * TPW * (ORN_RDC / 4)];
-                // Each quad's LDS reads are issued before the previous
-                // quad's arithmetic (two register sets; the empty asm keeps
-                // the reads above it and the arithmetic below it): 78 ->
-                // 71-74 us at 2048 tokens.  Groups of two quads ran 74-77,
-                // and of four took a wave per SIMD in registers.
-                constexpr int RG = 1, NG = ORN_RDC / 4 / RG;
-                v4f wA[RG], wB[RG], xA[TPW][RG], xB[TPW][RG];
-                auto rd = [&](v4f (&w)[RG], v4f (&xv)[TPW][RG], int g) {
+                // The first NB tokens' values are read from LDS as a
+                // broadcast, quad by quad; of the others a lane takes four of
+                // the 64 with one read and gets the rest from its row of 16
+                // lanes (row_newbcast in the multiply itself).  Each quad's
+                // reads are issued before the previous quad's arithmetic.
+                v4f xv[TPW], xq[2][NB > 0 ? NB : 1];
 #pragma unroll
-                    for (int q = 0; q < RG; ++q) {
-                        w[q] = wr[RG * g + q];
+                for (int j = NB; j < TPW; ++j) xv[j] = xr[j * (ORN_RDC / 4) + (lane & 15)];
+                v4f w2[2];
+                w2[0] = wr[0];
 #pragma unroll
-                        for (int j = 0; j < TPW; ++j) xv[j][q] = xr[j * (ORN_RDC / 4) + RG * g + q];
+                for (int j = 0; j < NB; ++j) xq[0][j] = xr[j * (ORN_RDC / 4)];
+                auto quad = [&](auto gc) {
+                    constexpr int G = decltype(gc)::value;
+                    if constexpr (G + 1 < ORN_RDC / 4) {
+                        w2[(G + 1) & 1] = wr[G + 1];
+#pragma unroll
+                        for (int j = 0; j < NB; ++j) xq[(G + 1) & 1][j] = xr[j * (ORN_RDC / 4) + G + 1];
                     }
-                };
-                rd(wA, xA, 0);
-#pragma unroll
-                for (int g = 0; g < NG; ++g) {
-                    v4f(&wc)[RG] = (g & 1) ? wB : wA;
-                    v4f(&wn)[RG] = (g & 1) ? wA : wB;
-                    v4f(&xc)[TPW][RG] = (g & 1) ? xB : xA;
-                    v4f(&xn)[TPW][RG] = (g & 1) ? xA : xB;
-                    if (g + 1 < NG) rd(wn, xn, g + 1);
 #pragma unroll
                     for (int j = 0; j < TPW; ++j) asm volatile("" : "+v"(acc[j])::"memory");
+                    const v4f wv = w2[G & 1];
 #pragma unroll
-                    for (int q = 0; q < RG; ++q)
+                    for (int i = 0; i < 4; ++i)
 #pragma unroll
-                        for (int j = 0; j < TPW; ++j) {
-                            const v4f xv = xc[j][q], wv = wc[q];
-                            acc[j] = acc[j] + xv.x * wv.x;
-                            acc[j] = acc[j] + xv.y * wv.y;
-                            acc[j] = acc[j] + xv.z * wv.z;
-                            acc[j] = acc[j] + xv.w * wv.w;
-                        }
-                }
+                        for (int j = 0; j < TPW; ++j)
+                            acc[j] = acc[j] + (j < NB ? xq[G & 1][j < NB ? j : 0][i] : row_bcast<G>(xv[j][i])) * wv[i];
+                };
+                for_each_quad(quad, std::make_integer_sequence<int, ORN_RDC / 4>{});
             }
         }
     }
@@ -294,89 +302,6 @@ __global__ void __launch_bounds__(256)
         const int tt = tid / (ORN_RDC / 4), t = t0 + tt;
         if (xon[0] && tid % (ORN_RDC / 4) == 0 && t < T) amax[t] = xmax;
     }
-}
-
-// ---------------------------------------------------------------------------
-// MoE router logits, few tokens (decode).  Block = one wave = one token over
-// 64 experts (lane = expert), so the 2 MiB router streams through 4*T CUs.
-// A lane's weights for quad d4 are the 16 bytes at Wq[d4][e][0..3], so one
-// wave load instruction reads 1 KB contiguous.  The loads run ORN_DPF quads
-// ahead in a register ring (branch-free, fully unrolled); the token's
-// activation row sits in LDS and is read as a broadcast.
-// ---------------------------------------------------------------------------
-#define ORN_DPF 8  // weight quads in flight per lane
-
-// Orders LDS accesses of the lanes of one wave across this point (the wave's
-// LDS operations execute in issue order; this keeps the compiler from
-// moving them).
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-__global__ void __launch_bounds__(64)
-    k_router_dec(const float *__restrict__ x, const float *__restrict__ Wq,
-                 const float *__restrict__ bias, int T, int D, int E,
-                 float *__restrict__ logits, int *ctl, float *__restrict__ amax)
-{
-    extern __shared__ v4f xsh[];  // [D/4]
-    const int lane = threadIdx.x;
-    const int e0 = blockIdx.x * 64;
-    const int t = blockIdx.y;
-    // The routing step is the first of every forward: clear its counters.
-    if (ctl && blockIdx.x == 0 && blockIdx.y == 0 && lane < 16) ctl[lane] = 0;
-    const int nd4 = D / 4;  // a multiple of ORN_DPF (checked by the launcher)
-    v4f *xw = xsh;
-    const v4f *xg = reinterpret_cast<const v4f *>(x + (size_t)t * D);
-    {
-        // All loads first, then the LDS writes (D <= 4096: at most 16 per lane).
-        v4f tmp[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j)
-            if (lane + 64 * j < nd4) tmp[j] = xg[lane + 64 * j];
-#pragma unroll
-        for (int j = 0; j < 16; ++j)
-            if (lane + 64 * j < nd4) xw[lane + 64 * j] = tmp[j];
-        // max |x| of the row for the MFMA activation scaling (block column 0)
-        if (amax && blockIdx.x == 0) {
-            float mx = 0.0f;
-#pragma unroll
-            for (int j = 0; j < 16; ++j)
-                if (lane + 64 * j < nd4)
-                    mx = fmaxf(mx, fmaxf(fmaxf(fabsf(tmp[j].x), fabsf(tmp[j].y)),
-                                         fmaxf(fabsf(tmp[j].z), fabsf(tmp[j].w))));
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-            if (lane == 0) amax[t] = mx;
-        }
-    }
-    wave_sync();
-
-    const int e = min(e0 + lane, E - 1);  // lanes past E compute a copy, never stored
-    const v4f *wp = reinterpret_cast<const v4f *>(Wq) + e;  // quad d4 at wp[d4*E]
-    v4f r[ORN_DPF];
-#pragma unroll
-    for (int p = 0; p < ORN_DPF; ++p) r[p] = wp[(size_t)p * E];
-    float acc = 0.0f;
-    for (int i0 = 0; i0 < nd4; i0 += ORN_DPF) {
-        v4f xv4[ORN_DPF];  // this iteration's activations, read up front
-#pragma unroll
-        for (int p = 0; p < ORN_DPF; ++p) xv4[p] = xw[i0 + p];
-#pragma unroll
-        for (int p = 0; p < ORN_DPF; ++p) {
-            // Use the slot, then refill it: the refill reuses its registers.
-            const v4f xv = xv4[p];
-            acc = acc + xv.x * r[p].x;
-            acc = acc + xv.y * r[p].y;
-            acc = acc + xv.z * r[p].z;
-            acc = acc + xv.w * r[p].w;
-            r[p] = wp[(size_t)min(i0 + p + ORN_DPF, nd4 - 1) * E];
-            __builtin_amdgcn_sched_barrier(0);  // keep the refill here, ORN_DPF quads ahead
-        }
-    }
-    if (e0 + lane < E) logits[(size_t)t * E + e0 + lane] = bias ? acc + bias[e0 + lane] : acc;
 }
 
 // ---------------------------------------------------------------------------
@@ -684,8 +609,8 @@ extern "C" int ornk_moe_route(const ornk_moe_args *a, hipStream_t s)
 {
     const int T = a->T, D = a->D, E = a->E;
     if (T <= 0) return hipSuccess;
-    if (E < 1 || E > 256 || a->k < 1 || a->k > 16 || a->k > E || D % (4 * ORN_DPF) ||
-        D % (ORN_RDC * ORN_RPF) || D > 4096)
+    if (E < 1 || E > 256 || a->k < 1 || a->k > 16 || a->k > E || D % (ORN_RDC * ORN_RPF) ||
+        D > 4096)
         return hipErrorInvalidValue;
     const float *xin = a->apply_norm ? a->xn : a->x;
     float *amax = a->router_amax ? a->x_amax : nullptr;  // every routing kernel can write it
@@ -707,18 +632,23 @@ extern "C" int ornk_moe_route(const ornk_moe_args *a, hipStream_t s)
         default: ORN_RPC(128); break;
         }
 #undef ORN_RPC
-    } else if (T >= 1024) {
-        ORN_LAUNCH_EV(a, k_router_seq<4>, dim3((E + 63) / 64, (T + 15) / 16), dim3(256), 0, s,
-                           xin, a->router, a->bias, T, D, E, a->logits, a->ctl, amax);
-    } else if (T >= 384) {
-        // 4 tokens per block: enough blocks for every CU (measured at 512
-        // tokens: 36.5 us against 49.5 us for k_router_dec; at 256, 31 us
-        // against 25-34 us)
-        ORN_LAUNCH_EV(a, k_router_seq<1>, dim3((E + 63) / 64, (T + 3) / 4), dim3(256), 0, s,
-                           xin, a->router, a->bias, T, D, E, a->logits, a->ctl, amax);
     } else {
-        ORN_LAUNCH_EV(a, k_router_dec, dim3((E + 63) / 64, T), dim3(64), sizeof(float) * (size_t)D,
-                           s, xin, a->router, a->bias, T, D, E, a->logits, a->ctl, amax);
+        // Tokens per wave: one, their values broadcast by the multiplies,
+        // while that leaves a SIMD few waves (the multiply takes twice the
+        // issue time, the LDS reads it replaces are shared by every wave of
+        // the CU); then two, then four, broadcast from LDS.  us with one / two
+        // / four: 300 tokens 29 / - / -, 512 32 / 37 / 52, 1000 54 / 45 / 56,
+        // 1500 77 / 61 / 64, 2048 94 / 75 / 67.  (Up to 383 tokens each wave
+        // streamed the router from L2 before: 31 us at 65, 34 at 300.)
+        const int tpw = T < 640 ? 1 : T < 1536 ? 2 : 4;
+        const dim3 gs((E + 63) / 64, (T + 4 * tpw - 1) / (4 * tpw));
+#define ORN_RSEQ(TPW, NB)                                                                        \
+    ORN_LAUNCH_EV(a, (k_router_seq<TPW, NB>), gs, dim3(256), 0, s, xin, a->router, a->bias, T, D, E, \
+                  a->logits, a->ctl, amax)
+        if (tpw == 1) ORN_RSEQ(1, 0);
+        else if (tpw == 2) ORN_RSEQ(2, 1);
+        else ORN_RSEQ(4, 4);
+#undef ORN_RSEQ
     }
     return hipGetLastError();
 }

@@ -5,9 +5,9 @@ a sequential fp32 sum from 0 of the fp32 products x[d]*W[d*E+e], d
 ascending, then + bias), so the logits it selected on must equal the
 oracle's (oracle/oracle.c orc_router_logits) as uint32, for every kernel
 instance the forward picks:
-  - k_router_pc (T <= 64), with its fused rmsnorm when ORN_MOE_NORM is set;
-  - k_router_dec (64 < T < 1024), after the separate rmsnorm kernel;
-  - k_router_seq (T >= 1024);
+  - k_router_pc (T <= 40), with its fused rmsnorm when ORN_MOE_NORM is set;
+  - k_router_seq (above, one, two or four tokens per wave), after the
+    separate rmsnorm kernel;
 with and without a Zipf router bias, and for the file-orientation store
 (router transposed at upload).  A one-ulp difference from a changed add
 order fails these tests, where index equality alone would not see it.
@@ -124,6 +124,15 @@ def test_router_dec_logits_bit_exact(om, ctx, store, T, norm):
 def test_router_seq_logits_bit_exact(om, ctx, store, T):
     """LDS-staged chains: 4 tokens per block (T < 1024), 16 (T >= 1024)."""
     check(om, ctx, store, T, 0, T == 400)
+
+
+@pytest.mark.parametrize("norm", [False, True], ids=["x", "rmsnorm"])
+@pytest.mark.parametrize("T", [40, 41, 43, 639, 640, 647, 1535, 1536])
+def test_router_instance_boundaries_bit_exact(om, ctx, store, T, norm):
+    """The step from the producer/consumer router to the staged one (40 / 41)
+    and between its instances of one, two and four tokens per wave, with work
+    groups whose last tokens are missing."""
+    check(om, ctx, store, T, 0, norm)
 
 
 @pytest.mark.parametrize("T", [1, 16, 256])
