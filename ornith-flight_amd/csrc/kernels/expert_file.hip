@@ -43,6 +43,8 @@
 #include "launch.h"
 #include "mfma_ops.h"
 
+#include <type_traits>
+
 using namespace orn_mfma;
 
 namespace {
@@ -352,14 +354,95 @@ __global__ void __launch_bounds__(256, 2)
 // ---------------------------------------------------------------------------
 #define ORN_FDN 2  // column tiles per wave in the down kernel
 
-template <int RT>
+// KSG > 0 (16-row items): each work group forms its rows' 256 values of mid
+// per super-block itself from the KSG gate/up partials (the mid step's order
+// and SiLU rules, k_mid_wg), scaled by the row's largest over the super-block
+// (a power of two, taken out again with d); mh, ml, minv are then not read.
+struct FileMid {
+    float v[16][256];
+    unsigned int amax[16];
+    float inv[16];
+};
+
+template <int KSG>
+__device__ __forceinline__ void form_mid(FileMid &M, FileTile &As, const float *__restrict__ gu,
+                                         int row0, int nr, int H, int s, int rows_max,
+                                         int shared_rows)
+{
+    constexpr int MG = 16 / KSG;  // rows whose partials are in flight together
+    const int tid = threadIdx.x, lane = tid & 63;
+    const size_t sstr = (size_t)rows_max * 2 * H;
+    if (tid < 16) M.amax[tid] = 0u;
+    __syncthreads();  // and every wave is done with the last super-block's tile
+    for (int r0 = 0; r0 < nr; r0 += MG) {
+        float gv[MG][KSG], uv[MG][KSG];
+#pragma unroll
+        for (int i = 0; i < MG; ++i) {
+            const float *p = gu + (size_t)(row0 + min(r0 + i, nr - 1)) * 2 * H + 256 * s + tid;
+#pragma unroll
+            for (int j = 0; j < KSG; ++j) {
+                gv[i][j] = p[j * sstr];
+                uv[i][j] = p[j * sstr + H];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < MG; ++i) {
+            const int r = r0 + i;
+            if (r >= nr) break;  // uniform
+            float g = 0.0f, u = 0.0f;
+#pragma unroll
+            for (int j = 0; j < KSG; ++j) {
+                g = g + gv[i][j];
+                u = u + uv[i][j];
+            }
+            float act;
+            if (row0 + r < shared_rows) {
+                act = g / (1.0f + expf(-g));
+            } else {
+                if (g < -50.0f) act = 0.0f;
+                else if (g > 50.0f) act = g;
+                else act = g / (1.0f + expf(-g));
+            }
+            const float v = act * u;
+            M.v[r][tid] = v;
+            float m = fabsf(v);
+#pragma unroll
+            for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+            // non-negative floats order like their bit patterns
+            if (lane == 0) atomicMax(&M.amax[r], __float_as_uint(m));
+        }
+    }
+    __syncthreads();
+    const int r = tid >> 4;  // 16 values of one row per thread
+    if (r < nr) {
+        const float sc = prep_scale(__uint_as_float(M.amax[r]));
+        if ((tid & 15) == 0) M.inv[r] = 1.0f / sc;
+#pragma unroll
+        for (int o = 0; o < 2; ++o) {
+            const int k = 16 * (tid & 15) + 8 * o;
+            const v4f a = *reinterpret_cast<const v4f *>(&M.v[r][k]) * sc;
+            const v4f b = *reinterpret_cast<const v4f *>(&M.v[r][k + 4]) * sc;
+            uint32_t h[4], l[4];
+            split2(a.x, a.z, h[0], l[0]);
+            split2(a.y, a.w, h[1], l[1]);
+            split2(b.x, b.z, h[2], l[2]);
+            split2(b.y, b.w, h[3], l[3]);
+            *reinterpret_cast<uint4 *>(&As.v[0][r][k]) = make_uint4(h[0], h[1], h[2], h[3]);
+            *reinterpret_cast<uint4 *>(&As.v[1][r][k]) = make_uint4(l[0], l[1], l[2], l[3]);
+        }
+    }
+    __syncthreads();
+}
+
+template <int RT, int KSG>
 __global__ void __launch_bounds__(256)
     k_dn_file(const uint8_t *__restrict__ body, const uint16_t *__restrict__ dv,
               const uint32_t *__restrict__ mh, const uint32_t *__restrict__ ml,
               const float *__restrict__ minv, const int *__restrict__ ctl,
               const int4 *__restrict__ items, float *__restrict__ dn, int D, int H, int ks,
-              int rows_max)
+              int rows_max, const float *__restrict__ gu, int shared_rows)
 {
+    static_assert(KSG == 0 || RT == 1, "mid is formed in the kernel for 16-row items only");
     const int NCB = D / (64 * ORN_FDN);
     const int per_item = NCB * ks;
     const int n_live = ctl[1] * per_item;
@@ -374,8 +457,9 @@ __global__ void __launch_bounds__(256)
     const size_t b0 = ((size_t)itm.w * D + n0) * NSB;  // first block of row n0
     const int nrows = itm.z;
     const int nrt = RT == 1 ? 1 : (nrows + 15) >> 4;
-    constexpr int NB = RT == 1 ? 2 : 1;
+    constexpr int NB = RT == 1 && !KSG ? 2 : 1;
     __shared__ __align__(16) FileTileT<RT> Ab[NB];  // A row = 16rt + c (mid rows)
+    __shared__ __align__(16) std::conditional_t<(KSG > 0), FileMid, int> M[1];
     __shared__ int src[16 * RT];
     if (threadIdx.x < 16 * RT)
         src[threadIdx.x] = itm.y + ((int)threadIdx.x < nrows ? (int)threadIdx.x : nrows - 1);
@@ -415,7 +499,10 @@ __global__ void __launch_bounds__(256)
                 qb[hn][ct] = *reinterpret_cast<const uint2 *>(blk[ct] + 128 + 32 * hn + 8 * g);
             }
         FileTileT<RT> &As = Ab[NB == 2 ? (s & 1) : 0];
-        stage_tile<RT, true>(As, mh, ml, src, H, s, nrows);
+        if constexpr (KSG > 0)
+            form_mid<KSG>(M[0], As, gu, itm.y, nrows, H, s, rows_max, shared_rows);
+        else
+            stage_tile<RT, true>(As, mh, ml, src, H, s, nrows);
         v4f ps[RT][ORN_FDN];  // this super-block's sums, before d
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt)
@@ -477,7 +564,12 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
             for (int ct = 0; ct < ORN_FDN; ++ct)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) acc[rt][ct][r] = fmaf(d[ct], ps[rt][ct][r], acc[rt][ct][r]);
+                for (int r = 0; r < 4; ++r) {
+                    const int row = 4 * g + r;  // past the item's rows: not stored
+                    float f = d[ct];
+                    if constexpr (KSG > 0) f *= row < nrows ? M[0].inv[row] : 0.0f;
+                    acc[rt][ct][r] = fmaf(f, ps[rt][ct][r], acc[rt][ct][r]);
+                }
     }
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
@@ -488,7 +580,8 @@ __global__ void __launch_bounds__(256)
             for (int r = 0; r < 4; ++r) {
                 const int row = 16 * rt + 4 * g + r;
                 if (row < nrows)
-                    out[(size_t)(4 * g + r) * D + 16 * ct] = acc[rt][ct][r] * minv[itm.y + row];
+                    out[(size_t)(4 * g + r) * D + 16 * ct] =
+                        KSG ? acc[rt][ct][r] : acc[rt][ct][r] * minv[itm.y + row];
             }
     }
 }
@@ -534,6 +627,14 @@ extern "C" int ornk_file_gateup(const ornk_moe_args *a, hipStream_t s)
     return hipGetLastError();
 }
 
+// The mid step's launch costs 4.1 us; formed here, by every work group of an
+// item, its values cost 1.3 us at one token (down 6.3 -> 7.6), 3.3 at four,
+// 5.7 at eight and 8 from 16 on.
+extern "C" int ornk_file_down_fuses_mid(int T, int tchunk, int ks_gu)
+{
+    return T <= 4 && tchunk == 16 && (ks_gu == 4 || ks_gu == 8);
+}
+
 extern "C" int ornk_file_down(const ornk_moe_args *a, hipStream_t s)
 {
     if (!ornk_file_supported(a->D, a->H) || (a->H / 256) % a->ks_dn) return hipErrorInvalidValue;
@@ -541,13 +642,14 @@ extern "C" int ornk_file_down(const ornk_moe_args *a, hipStream_t s)
     if (a->D % (64 * ORN_FDN)) return hipErrorInvalidValue;
     const dim3 grid(a->items_max * (a->D / (64 * ORN_FDN)) * a->ks_dn);
     if (a->tchunk > 64) return hipErrorInvalidValue;
-    if (a->tchunk > 16)
-        ORN_LAUNCH_EV(a, k_dn_file<4>, grid, dim3(256), 0, s, a->down_body, a->down_d, f.mh, f.ml,
-                      f.minv, a->ctl, reinterpret_cast<const int4 *>(a->items), a->dn_part, a->D,
-                      a->H, a->ks_dn, a->rows_max);
-    else
-        ORN_LAUNCH_EV(a, k_dn_file<1>, grid, dim3(256), 0, s, a->down_body, a->down_d, f.mh, f.ml,
-                      f.minv, a->ctl, reinterpret_cast<const int4 *>(a->items), a->dn_part, a->D,
-                      a->H, a->ks_dn, a->rows_max);
+#define ORN_DNF(R, K)                                                                            \
+    ORN_LAUNCH_EV(a, (k_dn_file<R, K>), grid, dim3(256), 0, s, a->down_body, a->down_d, f.mh, f.ml, \
+                  f.minv, a->ctl, reinterpret_cast<const int4 *>(a->items), a->dn_part, a->D, a->H, \
+                  a->ks_dn, a->rows_max, a->gu_part, a->has_shared ? a->T : 0)
+    if (a->tchunk > 16) ORN_DNF(4, 0);
+    else if (!ornk_file_down_fuses_mid(a->T, a->tchunk, a->ks_gu)) ORN_DNF(1, 0);
+    else if (a->ks_gu == 8) ORN_DNF(1, 8);
+    else ORN_DNF(1, 4);
+#undef ORN_DNF
     return hipGetLastError();
 }

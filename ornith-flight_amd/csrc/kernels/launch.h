@@ -268,6 +268,8 @@ int ornk_file_supported(int D, int H);
 int ornk_file_down_cols(void);
 int ornk_file_prep_x(const ornk_moe_args *a, hipStream_t s);
 int ornk_file_gateup(const ornk_moe_args *a, hipStream_t s);
+/* 1 if ornk_file_down forms mid from ks_gu gate/up partials itself. */
+int ornk_file_down_fuses_mid(int T, int tchunk, int ks_gu);
 int ornk_file_down(const ornk_moe_args *a, hipStream_t s);
 int ornk_rowmax(const float *x, int rows, int D, float *out, hipEvent_t start, hipStream_t s);
 int ornk_moe_combine(const ornk_moe_args *a, hipStream_t s);

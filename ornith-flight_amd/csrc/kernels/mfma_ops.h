@@ -167,4 +167,45 @@ __device__ __forceinline__ float prep_scale(float amax)
     return ldexpf(1.0f, e);
 }
 
+// One prepared row of the file-orientation activations by a work group of 256
+// threads: the row's D values in LDS, m = max |value|, r its number; hi/lo of
+// value * s in the pair order [0,2,1,3,4,6,5,7] of each 8, inv = 1/s and the
+// 32-value sub-block sums / 32 (expert_file.hip's k_prep_rows).
+template <int D>
+__device__ __forceinline__ void file_prep_row(const float *row, float m, int r, uint32_t *hi,
+                                              uint32_t *lo, float *inv, uint16_t *shi, uint16_t *slo)
+{
+    const float s = prep_scale(m);
+#pragma unroll
+    for (int g0 = 0; g0 < D / 8; g0 += 256) {
+        const int g = g0 + (int)threadIdx.x;  // group of 8 values
+        const bool on = g < D / 8;
+        const v4f a = reinterpret_cast<const v4f *>(row)[on ? 2 * g : 0] * s;
+        const v4f b = reinterpret_cast<const v4f *>(row)[on ? 2 * g + 1 : 1] * s;
+        if (on) {
+            uint32_t h[4], l[4];
+            split2(a.x, a.z, h[0], l[0]);
+            split2(a.y, a.w, h[1], l[1]);
+            split2(b.x, b.z, h[2], l[2]);
+            split2(b.y, b.w, h[3], l[3]);
+            const size_t o = (size_t)r * (D >> 1) + 4 * g;  // u32 words
+            *reinterpret_cast<uint4 *>(hi + o) = make_uint4(h[0], h[1], h[2], h[3]);
+            *reinterpret_cast<uint4 *>(lo + o) = make_uint4(l[0], l[1], l[2], l[3]);
+        }
+        // 4 consecutive threads hold one 32-value sub-block
+        float t = ((a.x + a.y) + (a.z + a.w)) + ((b.x + b.y) + (b.z + b.w));
+        t += __shfl_xor(t, 1, 64);
+        t += __shfl_xor(t, 2, 64);
+        if (on && (g & 3) == 0) {
+            t *= 0.03125f;
+            const _Float16 th = (_Float16)t;
+            const _Float16 tl = (_Float16)(t - (float)th);
+            const size_t o = (size_t)r * (D >> 5) + (g >> 2);
+            shi[o] = __builtin_bit_cast(uint16_t, th);
+            slo[o] = __builtin_bit_cast(uint16_t, tl);
+        }
+    }
+    if (threadIdx.x == 0) inv[r] = 1.0f / s;
+}
+
 }  // namespace orn_mfma

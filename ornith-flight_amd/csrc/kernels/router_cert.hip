@@ -92,7 +92,8 @@ struct CertArgs {
     int *ctl, *slot_expert, *slot_off, *slot_cnt, *row_token, *pair_row;
     int4 *items;
     int T, E, k, mode, ep_lo, ep_n, has_shared, items_max, tchunk;
-    int ngroups;  // expert work groups (with the rmsnorm, one more group runs its chain)
+    int ngroups;  // expert work groups (with the rmsnorm or fx, one more group)
+    ornk_file_ws fx;  // file-orientation stores: the rows' hi/lo activations (xh NULL: none)
 };
 
 __device__ __forceinline__ double readlane_d(double v, int l)
@@ -513,46 +514,59 @@ __global__ void __launch_bounds__(256) k_route_cert(CertArgs P)
     uint64_t *const inv_word = P.est + (size_t)T * E;  // [T] tagged rmsnorm scales
     const bool norm = P.norm_w != nullptr;
 
-    if (norm && eg == P.ngroups) {
-        // ---- the rmsnorm's group (gpu.c:144-156): the sequential sum of
-        // squares by lane 0 of wave t (the squares first, by every thread,
-        // so that the chain is adds only), then xn = w * (x * inv) and max
-        // |xn| for the expert steps, and inv for the selecting group ----
+    if ((norm || P.fx.xh) && eg == P.ngroups) {
+        // ---- the extra group.  The rmsnorm (gpu.c:144-156): the sequential
+        // sum of squares by lane 0 of wave t (the squares first, by every
+        // thread, so that the chain is adds only), then xn = w * (x * inv)
+        // and max |xn| for the expert steps, and inv for the selecting group.
+        // For a file-orientation store also its expert steps' activations
+        // (k_prep_rows' values; a launch of their own took 4 us) ----
         __shared__ float inv_s[CERT_TPG];
         v4f *sq = U.sq;
         for (int i = tid; i < nt * (D / 4); i += 256) {
             const int t = i / (D / 4), c = i % (D / 4);
             const v4f v = reinterpret_cast<const v4f *>(P.x + (size_t)(t0 + t) * D)[c];
             reinterpret_cast<v4f *>(xs[t])[c] = v;
-            sq[i] = v * v;
+            if (norm) sq[i] = v * v;
         }
         __syncthreads();
-        if (wave < nt && lane == 0) {
-            const float ss = orn_lds_seq_sum32_n<D / 32>(sq + wave * (D / 4));
-            inv_s[wave] = 1.0f / sqrtf(ss / (float)D + 1e-6f);
+        if (norm) {
+            if (wave < nt && lane == 0) {
+                const float ss = orn_lds_seq_sum32_n<D / 32>(sq + wave * (D / 4));
+                inv_s[wave] = 1.0f / sqrtf(ss / (float)D + 1e-6f);
+            }
+            __syncthreads();
+            if (tid < nt)
+                st_word(&inv_word[t0 + tid],
+                        ((uint64_t)__float_as_uint(inv_s[tid]) << 32) | (uint64_t)tag);
         }
-        __syncthreads();
-        if (tid < nt)
-            st_word(&inv_word[t0 + tid],
-                    ((uint64_t)__float_as_uint(inv_s[tid]) << 32) | (uint64_t)tag);
         for (int t = 0; t < nt; ++t) {
             float mx = 0.0f;
             for (int c = tid; c < D / 4; c += 256) {
-                const v4f wn = reinterpret_cast<const v4f *>(P.norm_w)[c];
-                const v4f v = wn * (reinterpret_cast<const v4f *>(xs[t])[c] * inv_s[t]);
-                reinterpret_cast<v4f *>(P.xn + (size_t)(t0 + t) * D)[c] = v;
+                v4f v = reinterpret_cast<const v4f *>(xs[t])[c];
+                if (norm) {
+                    const v4f wn = reinterpret_cast<const v4f *>(P.norm_w)[c];
+                    v = wn * (v * inv_s[t]);
+                    reinterpret_cast<v4f *>(P.xn + (size_t)(t0 + t) * D)[c] = v;
+                    if (P.fx.xh) reinterpret_cast<v4f *>(xs[t])[c] = v;
+                }
                 mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
             }
-            if (P.x_amax) {
 #pragma unroll
-                for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-                if (lane == 0) mx_s[t][wave] = mx;
-            }
+            for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+            if (lane == 0) mx_s[t][wave] = mx;
         }
         __syncthreads();
         if (P.x_amax && tid < nt)
             P.x_amax[t0 + tid] =
                 fmaxf(fmaxf(mx_s[tid][0], mx_s[tid][1]), fmaxf(mx_s[tid][2], mx_s[tid][3]));
+        if (P.fx.xh) {
+            for (int t = 0; t < nt; ++t) {
+                const float mx = fmaxf(fmaxf(mx_s[t][0], mx_s[t][1]), fmaxf(mx_s[t][2], mx_s[t][3]));
+                orn_mfma::file_prep_row<D>(xs[t], mx, t0 + t, P.fx.xh, P.fx.xl, P.fx.xinv, P.fx.xsh,
+                                           P.fx.xsl);
+            }
+        }
         return;
     }
 
@@ -572,7 +586,7 @@ __global__ void __launch_bounds__(256) k_route_cert(CertArgs P)
         reinterpret_cast<v4f *>(xs[t])[c] = v;
     }
     __syncthreads();
-    if (P.x_amax && eg == 0 && !norm) {
+    if (P.x_amax && eg == 0 && !norm) {  // (file stores take none)
         // max |x| per token for the MFMA activation scaling
         for (int t = 0; t < nt; ++t) {
             float mx = 0.0f;
@@ -847,7 +861,8 @@ extern "C" int ornk_moe_route_cert(const ornk_moe_args *a, hipStream_t s)
     P.items_max = a->items_max;
     P.tchunk = a->tchunk;
     P.ngroups = (E + CERT_EPG - 1) / CERT_EPG;
-    const dim3 grid(P.ngroups + (P.norm_w ? 1 : 0));  // + the rmsnorm's group
+    P.fx = a->fw;
+    const dim3 grid(P.ngroups + (P.norm_w || P.fx.xh ? 1 : 0));  // + the extra group
     switch (D / 256) {
     case 1: ORN_LAUNCH_EV(a, k_route_cert<1>, grid, dim3(256), 0, s, P); break;
     case 2: ORN_LAUNCH_EV(a, k_route_cert<2>, grid, dim3(256), 0, s, P); break;
