@@ -473,7 +473,7 @@ __device__ __forceinline__ int select_cert(float (&sfv)[4], float (&bfv)[4], boo
     return path;
 }
 
-template <int NQ>
+template <int NQ, bool FX>
 __global__ void __launch_bounds__(256) k_route_cert(CertArgs P)
 {
     constexpr int D = 256 * NQ, L = 4 * NQ;  // L: values per chunk (lane)
@@ -514,7 +514,7 @@ __global__ void __launch_bounds__(256) k_route_cert(CertArgs P)
     uint64_t *const inv_word = P.est + (size_t)T * E;  // [T] tagged rmsnorm scales
     const bool norm = P.norm_w != nullptr;
 
-    if ((norm || P.fx.xh) && eg == P.ngroups) {
+    if ((FX || norm) && eg == P.ngroups) {
         // ---- the extra group.  The rmsnorm (gpu.c:144-156): the sequential
         // sum of squares by lane 0 of wave t (the squares first, by every
         // thread, so that the chain is adds only), then xn = w * (x * inv)
@@ -527,10 +527,10 @@ __global__ void __launch_bounds__(256) k_route_cert(CertArgs P)
             const int t = i / (D / 4), c = i % (D / 4);
             const v4f v = reinterpret_cast<const v4f *>(P.x + (size_t)(t0 + t) * D)[c];
             reinterpret_cast<v4f *>(xs[t])[c] = v;
-            if (norm) sq[i] = v * v;
+            if (!FX || norm) sq[i] = v * v;
         }
         __syncthreads();
-        if (norm) {
+        if (!FX || norm) {
             if (wave < nt && lane == 0) {
                 const float ss = orn_lds_seq_sum32_n<D / 32>(sq + wave * (D / 4));
                 inv_s[wave] = 1.0f / sqrtf(ss / (float)D + 1e-6f);
@@ -544,23 +544,25 @@ __global__ void __launch_bounds__(256) k_route_cert(CertArgs P)
             float mx = 0.0f;
             for (int c = tid; c < D / 4; c += 256) {
                 v4f v = reinterpret_cast<const v4f *>(xs[t])[c];
-                if (norm) {
+                if (!FX || norm) {
                     const v4f wn = reinterpret_cast<const v4f *>(P.norm_w)[c];
                     v = wn * (v * inv_s[t]);
                     reinterpret_cast<v4f *>(P.xn + (size_t)(t0 + t) * D)[c] = v;
-                    if (P.fx.xh) reinterpret_cast<v4f *>(xs[t])[c] = v;
+                    if (FX) reinterpret_cast<v4f *>(xs[t])[c] = v;
                 }
                 mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
             }
+            if (FX || P.x_amax) {
 #pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-            if (lane == 0) mx_s[t][wave] = mx;
+                for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+                if (lane == 0) mx_s[t][wave] = mx;
+            }
         }
         __syncthreads();
         if (P.x_amax && tid < nt)
             P.x_amax[t0 + tid] =
                 fmaxf(fmaxf(mx_s[tid][0], mx_s[tid][1]), fmaxf(mx_s[tid][2], mx_s[tid][3]));
-        if (P.fx.xh) {
+        if constexpr (FX) {
             for (int t = 0; t < nt; ++t) {
                 const float mx = fmaxf(fmaxf(mx_s[t][0], mx_s[t][1]), fmaxf(mx_s[t][2], mx_s[t][3]));
                 orn_mfma::file_prep_row<D>(xs[t], mx, t0 + t, P.fx.xh, P.fx.xl, P.fx.xinv, P.fx.xsh,
@@ -586,7 +588,7 @@ __global__ void __launch_bounds__(256) k_route_cert(CertArgs P)
         reinterpret_cast<v4f *>(xs[t])[c] = v;
     }
     __syncthreads();
-    if (P.x_amax && eg == 0 && !norm) {  // (file stores take none)
+    if (P.x_amax && eg == 0 && !norm) {
         // max |x| per token for the MFMA activation scaling
         for (int t = 0; t < nt; ++t) {
             float mx = 0.0f;
@@ -862,14 +864,24 @@ extern "C" int ornk_moe_route_cert(const ornk_moe_args *a, hipStream_t s)
     P.tchunk = a->tchunk;
     P.ngroups = (E + CERT_EPG - 1) / CERT_EPG;
     P.fx = a->fw;
-    const dim3 grid(P.ngroups + (P.norm_w || P.fx.xh ? 1 : 0));  // + the extra group
+    // a store of file blocks has instances of its own, so that the others'
+    // code stays as it is (with one kernel for both, 0.25 us more at one token)
+    const bool fx = P.fx.xh != nullptr;
+    const dim3 grid(P.ngroups + (P.norm_w || fx ? 1 : 0));  // + the extra group
+#define ORN_RC(N)                                                                        \
+    if (fx) ORN_LAUNCH_EV(a, (k_route_cert<N, true>), grid, dim3(256), 0, s, P);         \
+    else ORN_LAUNCH_EV(a, (k_route_cert<N, false>), grid, dim3(256), 0, s, P)
     switch (D / 256) {
-    case 1: ORN_LAUNCH_EV(a, k_route_cert<1>, grid, dim3(256), 0, s, P); break;
-    case 2: ORN_LAUNCH_EV(a, k_route_cert<2>, grid, dim3(256), 0, s, P); break;
-    case 4: ORN_LAUNCH_EV(a, k_route_cert<4>, grid, dim3(256), 0, s, P); break;
-    case 8: ORN_LAUNCH_EV(a, k_route_cert<8>, grid, dim3(256), 0, s, P); break;
-    case 16: ORN_LAUNCH_EV(a, k_route_cert<16>, grid, dim3(256), 0, s, P); break;
+    case 1: ORN_RC(1); break;
+    case 2: ORN_RC(2); break;
+    case 4: ORN_RC(4); break;
+    case 8: ORN_RC(8); break;
+    case 16:  // file stores end at D = 2048
+        if (fx) return hipErrorInvalidValue;
+        ORN_LAUNCH_EV(a, (k_route_cert<16, false>), grid, dim3(256), 0, s, P);
+        break;
     default: return hipErrorInvalidValue;
     }
+#undef ORN_RC
     return hipGetLastError();
 }
