@@ -1074,7 +1074,9 @@ static plan_t make_plan_file(const ornith_moe_shape *sh, int T)
 /* MFMA kernels on vec@mat blocks: items of <= 16 rows up to 64 tokens, <= 32
  * above; the reduction is split so that gate/up and down have about 4096 work
  * groups of two waves (four rounds of the chip at their occupancy) but keep
- * slices of at least 4 steps.  0 if the shape's slices are not taken. */
+ * slices of at least 4 steps, and no more partials than the VALU kernels'
+ * plan (make_plan) where 64-step slices allow that, so that a batch that fits
+ * the fixed scratch with that one fits with this one.  0 if the shape's slices are not taken. */
 static int make_plan_blk(const ornith_moe_shape *sh, int T, plan_t *out)
 {
     plan_t p;
@@ -1091,6 +1093,13 @@ static int make_plan_blk(const ornith_moe_shape *sh, int T, plan_t *out)
     while (D / 32 / kg > 64) kg *= 2;
     while (kg > 1 && ((D / 32) % kg || D / 32 / kg < 4)) kg /= 2;
     while (kd > 1 && ((H / 32) % kd || H / 32 / kd < 4 || kd > 16)) kd /= 2;
+    const plan_t v = make_plan(sh, T, 0);
+    while (kg * 2 * H + kd * D > v.ks_gu * 2 * H + v.ks_dn * D) {
+        const int g = kg > 1 && D / 32 / (kg / 2) <= 64, d = kd > 1 && H / 32 / (kd / 2) <= 64;
+        if (g && (!d || kg * 2 * H >= kd * D)) kg /= 2;
+        else if (d) kd /= 2;
+        else break;
+    }
     p.ks_gu = kg;
     p.ks_dn = kd;
     if (!ornk_blk_supported(D / 32 / kg, H / 32 / kd)) return 0;
@@ -1124,6 +1133,53 @@ static int launch_k(gpu_context *ctx, const char *name,
     if (e != hipSuccess)
         return orn_set_err(ctx, ORN_EHIP, "%s: %s", name, hipGetErrorString((hipError_t)e));
     return ORN_OK;
+}
+
+/* The forward's work buffers: offsets from the workspace's start, which keeps
+ * `head` bytes for itself, and their end. */
+typedef struct {
+    size_t xn, est, logits, idx, w, ctl, slot_e, slot_off, slot_cnt, row_tok, pair_row, items;
+    size_t gu, mid, dn, xamax, midamax, fxh, fxl, fsh, fsl, fxinv, fmh, fml, fminv, end;
+} ws_t;
+
+static ws_t carve_ws(const ornith_moe_shape *sh, int T, const plan_t *p, int norm, int cert,
+                     int amax, size_t head)
+{
+    const int D = sh->d_model, H = sh->hidden, E = sh->n_experts, k = sh->top_k, E1 = E + 1;
+    const int file = sh->file_layout;
+    ws_t w;
+    size_t off = head;
+#define CARVE(name, bytes)  \
+    w.name = off;           \
+    off += ALIGN256((size_t)(bytes))
+    CARVE(xn, norm ? (size_t)T * D * 4 : 0);
+    CARVE(est, cert ? (size_t)T * (E + 1) * 8 : 0); /* tagged (S, B) words, rmsnorm scales */
+    CARVE(logits, (size_t)T * E * 4);
+    CARVE(idx, (size_t)T * k * 4);
+    CARVE(w, (size_t)T * k * 4);
+    CARVE(ctl, 64);
+    CARVE(slot_e, (size_t)E1 * 4);
+    CARVE(slot_off, (size_t)E1 * 4);
+    CARVE(slot_cnt, (size_t)E1 * 4);
+    CARVE(row_tok, (size_t)p->rows_max * 4);
+    CARVE(pair_row, (size_t)T * k * 4);
+    CARVE(items, (size_t)p->items_max * 16);
+    CARVE(gu, (size_t)p->ks_gu * p->rows_max * 2 * H * 4);
+    CARVE(mid, (size_t)p->rows_max * H * 4);
+    CARVE(dn, (size_t)p->ks_dn * p->rows_max * D * 4);
+    CARVE(xamax, amax ? (size_t)T * 4 : 0);
+    CARVE(midamax, amax ? (size_t)p->rows_max * 4 : 0);
+    CARVE(fxh, file ? (size_t)T * D * 2 : 0);
+    CARVE(fxl, file ? (size_t)T * D * 2 : 0);
+    CARVE(fsh, file ? (size_t)T * (D / 32) * 2 : 0);
+    CARVE(fsl, file ? (size_t)T * (D / 32) * 2 : 0);
+    CARVE(fxinv, file ? (size_t)T * 4 : 0);
+    CARVE(fmh, file ? (size_t)p->rows_max * H * 2 : 0);
+    CARVE(fml, file ? (size_t)p->rows_max * H * 2 : 0);
+    CARVE(fminv, file ? (size_t)p->rows_max * 4 : 0);
+#undef CARVE
+    w.end = off;
+    return w;
 }
 
 /* fixed_ws: NULL = the context's grow-only workspace; else the device's
@@ -1174,7 +1230,7 @@ static int moe_forward_dev(gpu_context *ctx, ornith_moe_store *st, int layer, co
     plan_t p;
     /* A store of blocks alone: the MFMA kernels that read them, unless the
      * call forces the VALU kernels. */
-    const int blk = !file && !mfma_ok && !(flags & ORN_MOE_PATH_VALU) && make_plan_blk(sh, T, &p);
+    int blk = !file && !mfma_ok && !(flags & ORN_MOE_PATH_VALU) && make_plan_blk(sh, T, &p);
     if (!blk) p = file ? make_plan_file(sh, T) : make_plan(sh, T, use_mfma);
 
     /* Certified routing of the smallest decode batches (router_cert.hip):
@@ -1182,54 +1238,38 @@ static int moe_forward_dev(gpu_context *ctx, ornith_moe_store *st, int layer, co
      * (the slot list is read back after the dispatch either way). */
     const int cert = !(flags & ORN_MOE_EXACT_LOGITS) && ornk_route_cert_supported(T, D, E, k);
 
+    const int norm = (flags & ORN_MOE_NORM) != 0;
+    if (blk) {
+        /* Its row maxima are a few bytes a row more than the VALU kernels'
+         * plan takes: at sizes where only that one fits the fixed scratch it
+         * runs, also in a call that may allocate (both give the same bits). */
+        const plan_t v = make_plan(sh, T, 0);
+        if (carve_ws(sh, T, &p, norm, cert, 1, ORNK_SYNC_BYTES).end > ORNK_SCRATCH_BYTES &&
+            carve_ws(sh, T, &v, norm, cert, 0, ORNK_SYNC_BYTES).end <= ORNK_SCRATCH_BYTES) {
+            blk = 0;
+            p = v;
+        }
+    }
+
     /* the fixed scratch keeps its first ORNK_SYNC_BYTES for the routing
      * counters (zeroed when the scratch is first resolved); otherwise they
      * have an allocation of their own */
-    size_t off = fixed_ws ? ORNK_SYNC_BYTES : 0;
     int *sync = NULL;
     if (cert) {
         sync = fixed_ws ? (int *)fixed_ws : ctx_sync(ctx);
         if (!sync) return ORN_ENOMEM;
     }
-#define CARVE(name, bytes)       \
-    size_t name = off;           \
-    off += ALIGN256((size_t)(bytes))
-    CARVE(o_xn, (flags & ORN_MOE_NORM) ? (size_t)T * D * 4 : 0);
-    CARVE(o_est, cert ? (size_t)T * (E + 1) * 8 : 0); /* tagged (S, B) words, rmsnorm scales */
-    CARVE(o_logits, (size_t)T * E * 4);
-    CARVE(o_idx, (size_t)T * k * 4);
-    CARVE(o_w, (size_t)T * k * 4);
-    CARVE(o_ctl, 64);
-    CARVE(o_slot_e, (size_t)E1 * 4);
-    CARVE(o_slot_off, (size_t)E1 * 4);
-    CARVE(o_slot_cnt, (size_t)E1 * 4);
-    CARVE(o_row_tok, (size_t)p.rows_max * 4);
-    CARVE(o_pair_row, (size_t)T * k * 4);
-    CARVE(o_items, (size_t)p.items_max * 16);
-    CARVE(o_gu, (size_t)p.ks_gu * p.rows_max * 2 * H * 4);
-    CARVE(o_mid, (size_t)p.rows_max * H * 4);
-    CARVE(o_dn, (size_t)p.ks_dn * p.rows_max * D * 4);
-    CARVE(o_xamax, use_mfma || blk ? (size_t)T * 4 : 0);
-    CARVE(o_midamax, use_mfma || blk ? (size_t)p.rows_max * 4 : 0);
-    CARVE(o_fxh, file ? (size_t)T * D * 2 : 0);
-    CARVE(o_fxl, file ? (size_t)T * D * 2 : 0);
-    CARVE(o_fsh, file ? (size_t)T * (D / 32) * 2 : 0);
-    CARVE(o_fsl, file ? (size_t)T * (D / 32) * 2 : 0);
-    CARVE(o_fxinv, file ? (size_t)T * 4 : 0);
-    CARVE(o_fmh, file ? (size_t)p.rows_max * H * 2 : 0);
-    CARVE(o_fml, file ? (size_t)p.rows_max * H * 2 : 0);
-    CARVE(o_fminv, file ? (size_t)p.rows_max * 4 : 0);
-#undef CARVE
+    const ws_t o = carve_ws(sh, T, &p, norm, cert, use_mfma || blk, fixed_ws ? ORNK_SYNC_BYTES : 0);
     uint8_t *ws;
     if (fixed_ws) {
-        if (off > ORNK_SCRATCH_BYTES)
+        if (o.end > ORNK_SCRATCH_BYTES)
             return orn_set_err(ctx, ORN_EINVAL,
                                "gpu_moe_forward_noalloc: %d tokens need %zu bytes of work "
                                "buffers; the fixed scratch holds %u",
-                               T, off, (unsigned)ORNK_SCRATCH_BYTES);
+                               T, o.end, (unsigned)ORNK_SCRATCH_BYTES);
         ws = (uint8_t *)fixed_ws;
     } else {
-        ws = (uint8_t *)orn_ws_get(ctx, off);
+        ws = (uint8_t *)orn_ws_get(ctx, o.end);
         if (!ws) return ORN_ENOMEM;
     }
 
@@ -1270,23 +1310,23 @@ static int moe_forward_dev(gpu_context *ctx, ornith_moe_store *st, int layer, co
     a.x = x;
     a.resid = resid;
     a.out = out;
-    a.xn = a.apply_norm ? (float *)(ws + o_xn) : (float *)x;
-    a.logits = (float *)(ws + o_logits);
+    a.xn = a.apply_norm ? (float *)(ws + o.xn) : (float *)x;
+    a.logits = (float *)(ws + o.logits);
     a.sync = sync;
-    a.route_est = cert ? (double *)(ws + o_est) : NULL;
+    a.route_est = cert ? (double *)(ws + o.est) : NULL;
     /* the selection is written straight into the caller's buffers if given */
-    a.idx = idx_out ? idx_out : (uint32_t *)(ws + o_idx);
-    a.w = w_out ? w_out : (float *)(ws + o_w);
-    a.ctl = (int *)(ws + o_ctl);
-    a.slot_expert = (int *)(ws + o_slot_e);
-    a.slot_off = (int *)(ws + o_slot_off);
-    a.slot_cnt = (int *)(ws + o_slot_cnt);
-    a.row_token = (int *)(ws + o_row_tok);
-    a.pair_row = (int *)(ws + o_pair_row);
-    a.items = (int *)(ws + o_items);
-    a.gu_part = (float *)(ws + o_gu);
-    a.mid = (float *)(ws + o_mid);
-    a.dn_part = (float *)(ws + o_dn);
+    a.idx = idx_out ? idx_out : (uint32_t *)(ws + o.idx);
+    a.w = w_out ? w_out : (float *)(ws + o.w);
+    a.ctl = (int *)(ws + o.ctl);
+    a.slot_expert = (int *)(ws + o.slot_e);
+    a.slot_off = (int *)(ws + o.slot_off);
+    a.slot_cnt = (int *)(ws + o.slot_cnt);
+    a.row_token = (int *)(ws + o.row_tok);
+    a.pair_row = (int *)(ws + o.pair_row);
+    a.items = (int *)(ws + o.items);
+    a.gu_part = (float *)(ws + o.gu);
+    a.mid = (float *)(ws + o.mid);
+    a.dn_part = (float *)(ws + o.dn);
     a.use_mfma = use_mfma || blk;
     a.q6_wide = st->q6_scmax && st->q6_scmax[layer] > 64; /* held by MFMA-layout stores */
     if (use_mfma && !st->cache) {  /* a streamed store's slot arrays come from the cache */
@@ -1305,20 +1345,20 @@ static int moe_forward_dev(gpu_context *ctx, ornith_moe_store *st, int layer, co
         a.dn_pf.dmax = st->dmax + slot0 * 3;
     }
     if (use_mfma || blk) {
-        a.x_amax = (float *)(ws + o_xamax);
+        a.x_amax = (float *)(ws + o.xamax);
         a.router_amax = 1;  /* every routing kernel writes the rows' max |x| */
-        a.mid_amax = (float *)(ws + o_midamax);
+        a.mid_amax = (float *)(ws + o.midamax);
     }
 
     if (file) {
-        a.fw.xh = (uint32_t *)(ws + o_fxh);
-        a.fw.xl = (uint32_t *)(ws + o_fxl);
-        a.fw.xsh = (uint16_t *)(ws + o_fsh);
-        a.fw.xsl = (uint16_t *)(ws + o_fsl);
-        a.fw.xinv = (float *)(ws + o_fxinv);
-        a.fw.mh = (uint32_t *)(ws + o_fmh);
-        a.fw.ml = (uint32_t *)(ws + o_fml);
-        a.fw.minv = (float *)(ws + o_fminv);
+        a.fw.xh = (uint32_t *)(ws + o.fxh);
+        a.fw.xl = (uint32_t *)(ws + o.fxl);
+        a.fw.xsh = (uint16_t *)(ws + o.fsh);
+        a.fw.xsl = (uint16_t *)(ws + o.fsl);
+        a.fw.xinv = (float *)(ws + o.fxinv);
+        a.fw.mh = (uint32_t *)(ws + o.fmh);
+        a.fw.ml = (uint32_t *)(ws + o.fml);
+        a.fw.minv = (float *)(ws + o.fminv);
     }
 
     int rc;

@@ -103,3 +103,24 @@ def test_blocks_mfma_row_isolation(om, ctx):
     perm = np.random.default_rng(1).permutation(T)
     assert np.array_equal(forward(om, ctx, st, x[perm], 0)[0], out[perm])
     st.close()
+
+
+# Batches that fit gpu_moe_forward_noalloc's 32 MiB with the fp32 kernels'
+# plan: the first two would not with slices for 4096 work groups (51 and 52
+# MB), the last misses by its row maxima and stays with the fp32 kernels.
+@pytest.mark.parametrize("D,H,E,k,shared,T,blk", [(2048, 512, 8, 8, False, 64, True),
+                                                  (1024, 1024, 8, 8, False, 64, True),
+                                                  (256, 256, 8, 8, True, 905, False)])
+def test_blocks_mfma_fixed_scratch(om, ctx, D, H, E, k, shared, T, blk):
+    st = om.Store(ctx, 1, D, H, E, k, shared, prefill_layout=False)
+    st.fill_synthetic(0, 5)
+    x = om.synth_normal(9, om.synth_stream(0, om.SYN_ACT, 0), T * D, 1.0).reshape(T, D)
+    names = []
+    ref = forward(om, ctx, st, x, 0, names=names)
+    assert ("moe_gateup_blk" in names) == blk
+    xb, ob = ctx.upload(x), ctx.alloc(x.nbytes)
+    st.forward(0, xb, T, ob, resid=xb, noalloc=True)
+    assert np.array_equal(ctx.download(ob, np.float32, x.shape), ref[0])
+    st.close()
+    for b in (xb, ob):
+        b.free()
