@@ -1,6 +1,7 @@
 // SPDX-License-Identifier: MIT
 //
-// Routed-MoE expert path on the vector ALUs (few tokens per expert):
+// Routed-MoE expert path on the vector ALUs (ORN_MOE_PATH_VALU, and block
+// stores whose shape or size the matrix-core kernels do not take):
 // fused Q4_K dequant-matvec for gate+up -> SiLU(gate)*up ->
 // Q6_K dequant-matvec for down -> weighted combine.  fp32 VALU arithmetic
 // (explicit fmaf), weights decoded in registers straight from the resident

@@ -8,9 +8,9 @@
 //
 // The MoE path computes every logit with exactly that arithmetic, one chain
 // per (token, expert), all chains in parallel (k_router_pc for decode-sized
-// batches, k_router_seq above), so the logits are
-// bit-identical to the reference's by construction.  Top-k selection and
-// the dispatch that follows it: dispatch.hip.
+// batches, k_router_seq above), so the logits are bit-identical to the
+// reference's by construction.  Top-k selection and the dispatch that follows
+// it: dispatch.hip.
 #include "common.h"
 #include "launch.h"
 #include "mfma_ops.h"
@@ -19,7 +19,6 @@
 #include <limits.h>
 
 #include <utility>
-
 
 namespace {
 
