@@ -635,8 +635,7 @@ def main():
             if close:
                 st.close()
 
-        # The fp32 VALU kernels on the headline layer (the path of a store
-        # kept without the MFMA layouts, and the reference-order fallback).
+        # The fp32 VALU kernels on the headline layer (ORN_MOE_PATH_VALU).
         if not args.only or args.only.startswith("valu_"):
             side_store("valu_", store, om.MOE_PATH_VALU, close=False)
         if not args.only or args.only.startswith("file_"):
