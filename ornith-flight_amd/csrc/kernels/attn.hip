@@ -146,7 +146,7 @@ __global__ __launch_bounds__(256) void k_attention(float *out, const float *Q, c
 //   out = O / L where the unshifted sum e^M L exceeds 1e-10, else O e^M
 // (attention.metal:60-62).
 // ---------------------------------------------------------------------------
-// Whether any of the operands is not finite (the same answer in every thread).
+// Whether any of the operands is not for the pairs (the same answer in every thread).
 __device__ __forceinline__ bool attn_bad(const int *bad, int ntq)
 {
     int b = 0;
@@ -350,8 +350,10 @@ __global__ void k_attn_merge(float *out, const float *Op, const float *mlp, int 
 // is hi*hi + hi*lo + lo*hi, what is dropped is below 2^-24 of it, and the sums
 // are fp32: the rounding of fp32 products at 3/16 of their matrix time.  The
 // pairs are made once per call (k_attn_prep), not once per work group.
-// Operands that hold a NaN or an infinity take k_attn_mma instead, decided on
-// the device (bad[]).
+// Operands that hold a NaN, an infinity or a value past 2^60 take k_attn_mma
+// instead, decided on the device (bad[]): below that the product of two rows'
+// scales is far from overflow, so a score of 0 stays 0 and every score that
+// is finite in fp32 stays finite.
 //
 // Work group: 4 waves of 32 query rows each and one split of the keys, tiles
 // of 32 keys.  Scores are formed transposed, S^T = K Q^T, so that a lane holds
@@ -370,12 +372,13 @@ __global__ void k_attn_merge(float *out, const float *Op, const float *mlp, int 
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 constexpr int AS_TK = 32, AS_ROWS = 128;  // keys per tile, query rows per work group
+constexpr float AS_MAX = 0x1p60f;           // largest operand the pairs take
 
 struct AttnPrep {
     _Float16 *q;      // [rows][hi, lo][HD]
     uint4 *kv;        // per tile [K hi][K lo] 32 x HD, [V hi][V lo] HD x 32
     float *qinv, *kinv, *vinv;
-    int *bad;         // [tiles][Q, K, V]: the tile's values are not all finite
+    int *bad;         // [tiles][Q, K, V]: not all of the tile's values are within AS_MAX
 };
 
 // Column maxima of V over a slice of rows: part[blockIdx.x][HD] (hd % 4 == 0).
@@ -454,7 +457,7 @@ __global__ void __launch_bounds__(256) k_attn_prep(AttnPrep P, const float *part
             float m = 0.0f;
 #pragma unroll
             for (int j = 0; j < W; ++j) {
-                ok = ok && fabsf(x[i][j]) <= 3.4028235e38f;
+                ok = ok && fabsf(x[i][j]) <= AS_MAX;
                 m = fmaxf(m, fabsf(x[i][j]));
             }
 #pragma unroll
@@ -503,7 +506,7 @@ __global__ void __launch_bounds__(256) k_attn_prep(AttnPrep P, const float *part
             v8h hi, lo;
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                ok = ok && fabsf(x[n][e]) <= 3.4028235e38f;
+                ok = ok && fabsf(x[n][e]) <= AS_MAX;
                 const float v = x[n][e] * vs[c];
                 hi[e] = (_Float16)v;
                 lo[e] = (_Float16)(v - (float)hi[e]);

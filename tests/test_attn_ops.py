@@ -224,6 +224,23 @@ def test_gpu_attention_pairs_not_finite(om, ctx):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("big,small", [(1e30, 1.0), (2.0 ** 60, 2.0 ** -60), (2.0 ** 61, 2.0 ** -61)])
+def test_gpu_attention_pairs_huge_operands(om, ctx, big, small):
+    """Rows of Q and K with huge values in columns that the other one leaves
+    at 0: the scores are the rest's, at any magnitude that fp32 holds (the
+    product of the rows' own scales would not be one).  Tolerance as for the
+    plain scores, whose products and sums these are."""
+    rng = np.random.default_rng(5)
+    seq, hd = 2180, 64
+    Q, K, V = (f32(rng.standard_normal((seq, hd))) for _ in range(3))
+    Q[:, 0], K[:, 0] = big, 0
+    Q[:, 1], K[:, 1] = 0, big
+    Q[:, 2:], K[:, 2:] = (0, 0) if small == 1.0 else (Q[:, 2:] * small, K[:, 2:] * small)
+    ref = attention64(Q, K, V)
+    assert np.abs(run_attention(om, ctx, Q, K, V) - ref).max() < 2e-6 * np.abs(ref).max()
+
+
+@pytest.mark.gpu
 def test_gpu_attention_large_scores(om, ctx):
     """Scores above 88: the shader's unshifted e^s overflows (the oracle
     gives NaN); the device returns the softmax."""
