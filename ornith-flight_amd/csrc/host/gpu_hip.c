@@ -321,11 +321,16 @@ void gpu_attention(gpu_context *ctx, gpu_buffer *out, const gpu_buffer *Q,
         return;
     }
     const float scale = 1.0f / sqrtf((float)head_dim);
-    if (head_dim % 4 == 0) {
-        /* matrix cores; the key splits' partials live in the context workspace */
-        const size_t wsb = ornk_attention_mma_ws(seq_len, head_dim);
-        void *ws = wsb ? orn_ws_get(ctx, wsb) : NULL;
-        if (wsb && !ws) return;
+    /* Matrix cores for head_dim % 4 == 0; the operand pairs and the key splits'
+     * partials live in the context workspace.  Where the card has no room for
+     * that, the kernel that needs none. */
+    const size_t wsb = head_dim % 4 == 0 ? ornk_attention_mma_ws(seq_len, head_dim) : 0;
+    void *ws = wsb ? orn_ws_get(ctx, wsb) : NULL;
+    if (wsb && !ws) {
+        (void)hipGetLastError(); /* the allocation's, which the launch would report */
+        ctx->err[0] = 0;
+    }
+    if (head_dim % 4 == 0 && (!wsb || ws)) {
         orn_hip_check(ctx, (hipError_t)ornk_attention_mma((float *)out->dev, (const float *)Q->dev,
                                                           (const float *)K_cache->dev,
                                                           (const float *)V_cache->dev, seq_len,
