@@ -346,10 +346,12 @@ __global__ void k_attn_merge(float *out, const float *Op, const float *mlp, int 
 //
 // Every operand is x * s = hi + lo, s a power of two per row of Q and of K and
 // per column of V (|x * s| < 2^14; 2^13 for the softmax weights), hi and
-// lo each rounded to nearest, so hi + lo holds x to 2^-24 of itself; a product
-// is hi*hi + hi*lo + lo*hi, what is dropped is below 2^-24 of it, and the sums
-// are fp32: the rounding of fp32 products at 3/16 of their matrix time.  The
-// pairs are made once per call (k_attn_prep), not once per work group.
+// lo each rounded to nearest, so hi + lo holds x to 2^-24 of itself or, where
+// fp16 has no smaller step, to 2^-38 of the largest value of its row or column;
+// a product is hi*hi + hi*lo + lo*hi, what is dropped is below 2^-24 of it, and
+// the sums are fp32: the rounding of fp32 products at 3/16 of their matrix
+// time.  The pairs are made once per call (k_attn_prep), not once per work
+// group.
 // Operands that hold a NaN, an infinity or a value past 2^60 take k_attn_mma
 // instead, decided on the device (bad[]): below that the product of two rows'
 // scales is far from overflow, so a score of 0 stays 0 and every score that
