@@ -960,15 +960,18 @@ static plan_t make_plan(const ornith_moe_shape *sh, int T, int use_mfma)
     const int D = sh->d_model, H = sh->hidden;
     /* MFMA work items hold at most one 16-row tile (the decode kernels) at
      * decode sizes, two (the decode kernels' two-tile instances) above 64
-     * tokens wherever the batch averages at most 32 rows per expert, four
-     * (the prefill grouped GEMMs) beyond: with 256 experts and top 8 the
-     * layer takes 288 / 324 us (two tiles / four) at 600 tokens, 340 / 362
-     * at 900, 369 / 381 at 1024, 389 / 391 at 1100, 497 / 425 at 1400.
+     * tokens wherever the batch averages at most 32 rows per expert (16 below
+     * 192 tokens: fewer experts then, whose gate/up slices of 16 steps would
+     * take more partials than the fixed scratch holds), four (the prefill
+     * grouped GEMMs) beyond: with 256 experts and top 8 the layer takes
+     * 288 / 324 us (two tiles / four) at 600 tokens, 340 / 362 at 900,
+     * 369 / 381 at 1024, 389 / 391 at 1100, 497 / 425 at 1400.
      * Skewed batches (a few hot experts, many cold ones) then split each
      * hot expert into items of 32 rows instead of running every cold expert
      * through a 64-row tile: an item costs its weight conversion whatever
      * its rows. */
-    p.tchunk = use_mfma ? (T <= 64 ? 16 : T * k <= 32 * E ? 32 : 64) : (T <= 64 ? 2 : 8);
+    const int two = T * k <= (T >= 192 ? 32 : 16) * E; /* two tiles */
+    p.tchunk = use_mfma ? (T <= 64 ? 16 : two ? 32 : 64) : (T <= 64 ? 2 : 8);
     p.rows_max = T * k + (sh->has_shared ? T : 0);
     const int max_slots = (T * k < E ? T * k : E) + (sh->has_shared ? 1 : 0);
     p.items_max = max_slots + (p.rows_max + p.tchunk - 1) / p.tchunk;

@@ -126,3 +126,22 @@ def test_noalloc_refuses_what_does_not_fit(om, ctx):
         assert np.array_equal(got[0].view(np.uint32), ref[0].view(np.uint32))
     finally:
         store.close()
+
+
+@pytest.mark.parametrize("E,k,T", [(104, 9, 185), (104, 10, 171), (104, 9, 195)])
+def test_noalloc_between_two_and_four_tiles(om, ctx, E, k, T):
+    """Batches of 16 to 32 rows per expert that fit the fixed scratch with
+    half the gate/up slices only (46 MB of work buffers otherwise at the first
+    two)."""
+    D, H = 2048, 512
+    store = om.Store(ctx, 1, D, H, E, k, False, prefill_layout=2)
+    try:
+        store.fill_synthetic(0, 5)
+        x = act(om, 37, T, D)
+        say(f"noalloc E={E} k={k} T={T}")
+        got = call(om, ctx, store, x, k, True)
+        ref = call(om, ctx, store, x, k, False)
+        for g, r in zip(got, ref):
+            assert np.array_equal(g.view(np.uint32), r.view(np.uint32))
+    finally:
+        store.close()
