@@ -1020,7 +1020,10 @@ static plan_t make_plan(const ornith_moe_shape *sh, int T, int use_mfma)
              * the chip with half as many work groups: the mid step then reads
              * half the partials (512 tokens gate/up 111 -> 105 us, mid 15 ->
              * 10; 709: 124 -> 114 and 20 -> 13; 128 tokens of a skewed batch
-             * 34.0 -> 35.1 and 5.1 -> 4.4) */
+             * 34.0 -> 35.1 and 5.1 -> 4.4).  The whole layer with 16 steps /
+             * 32: 200 tokens 213.7 / 209.3 us, 256 219.9 / 215.8; skewed, whose
+             * few experts leave less to fill the chip with, 200 136.8 / 139.4,
+             * 256 130.6 / 132.4, 350 170.6 / 167.7. */
             const int most = p.tchunk == 32 && T >= 192 ? 32 : 16;
             while ((D / 32) % (2 * dg) == 0 && D / 32 / dg > most) dg *= 2;
             int dd = 1;
