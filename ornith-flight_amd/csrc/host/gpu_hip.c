@@ -321,14 +321,17 @@ void gpu_attention(gpu_context *ctx, gpu_buffer *out, const gpu_buffer *Q,
         return;
     }
     const float scale = 1.0f / sqrtf((float)head_dim);
-    /* Matrix cores for head_dim % 4 == 0; the operand pairs and the key splits'
+    /* Matrix cores for head_dim % 4 == 0; the operands' parts and the key splits'
      * partials live in the context workspace.  Where the card has no room for
-     * that, the kernel that needs none. */
+     * that, the kernel that needs none; the call has not failed then, and the
+     * context keeps the error it had. */
     const size_t wsb = head_dim % 4 == 0 ? ornk_attention_mma_ws(seq_len, head_dim) : 0;
+    char err[sizeof ctx->err];
+    memcpy(err, ctx->err, sizeof err);
     void *ws = wsb ? orn_ws_get(ctx, wsb) : NULL;
     if (wsb && !ws) {
         (void)hipGetLastError(); /* the allocation's, which the launch would report */
-        ctx->err[0] = 0;
+        memcpy(ctx->err, err, sizeof err);
     }
     if (head_dim % 4 == 0 && (!wsb || ws)) {
         orn_hip_check(ctx, (hipError_t)ornk_attention_mma((float *)out->dev, (const float *)Q->dev,

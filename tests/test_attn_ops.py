@@ -18,6 +18,8 @@ above 88) the device still returns the softmax; that case is checked against
 fp64.
 """
 import ctypes as C
+import os
+import subprocess
 
 import numpy as np
 import pytest
@@ -93,6 +95,21 @@ def test_oracle_deltanet():
     assert np.array_equal(st1, S)
     st0, _ = O.deltanet_step(S, q, k, v, 0.0)
     assert np.array_equal(st0, f32(np.outer(v, k)))
+
+
+def test_attention_without_room_keeps_the_error(tmp_path):
+    """tests/attention_no_room.c: without room for the workspace gpu_attention
+    runs the kernel that needs none, and the context's error is what it was
+    before the call, read or not."""
+    here = os.path.dirname(os.path.abspath(__file__))
+    exe = tmp_path / "attention_no_room"
+    cmd = ["gcc", "-std=gnu99", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-no-pie",
+           "-Wl,--unresolved-symbols=ignore-all", "-o", str(exe),
+           os.path.join(here, "attention_no_room.c"), "-lm"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-3000:]
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60, check=True).stdout
+    assert out.split("\n")[:5] == ["", "", "an earlier call's error", "an earlier call's error", "2 0"]
 
 
 # ------------------------------------------------------------ GPU
