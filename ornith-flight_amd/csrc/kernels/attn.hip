@@ -4,7 +4,8 @@
 // dot-product attention, the gated DeltaNet step and the KV-cache append,
 // with the semantics of the reference's Metal kernels (ops.metal:113-139,
 // attention.metal:17-125) as dispatched by gpu_metal.m:495-583.  fp32
-// throughout, compiled with -ffp-contract=off.
+// operands and sums, compiled with -ffp-contract=off; the attention of long
+// sequences takes each fp32 operand as three bf16 parts.
 #include "common.h"
 #include "launch.h"
 
@@ -121,6 +122,15 @@ __global__ __launch_bounds__(256) void k_attention(float *out, const float *Q, c
     }
 }
 
+// Whether any of the operands is not to be split into parts, of ntq
+// tiles (k_attn_prep; the same answer in every thread).
+__device__ __forceinline__ bool attn_bad(const int *bad, int ntq)
+{
+    int b = 0;
+    for (int i = threadIdx.x; i < 3 * ntq; i += blockDim.x) b |= bad[i];
+    return __syncthreads_or(b) != 0;
+}
+
 // ---------------------------------------------------------------------------
 // The same attention on the matrix cores (v_mfma_f32_16x16x4f32: fp32 operands,
 // fp32 accumulation), for head dims that are a multiple of 4 (HD = 64, 128 or
@@ -146,14 +156,6 @@ __global__ __launch_bounds__(256) void k_attention(float *out, const float *Q, c
 //   out = O / L where the unshifted sum e^M L exceeds 1e-10, else O e^M
 // (attention.metal:60-62).
 // ---------------------------------------------------------------------------
-// Whether any of the operands is not for the pairs (the same answer in every thread).
-__device__ __forceinline__ bool attn_bad(const int *bad, int ntq)
-{
-    int b = 0;
-    for (int i = threadIdx.x; i < 3 * ntq; i += blockDim.x) b |= bad[i];
-    return __syncthreads_or(b) != 0;
-}
-
 constexpr int AM_TK = 16;  // keys per tile
 
 template <int HD>
@@ -170,7 +172,7 @@ __global__ void __launch_bounds__(256) k_attn_mma(float *out, float *Op, float *
                                                   const int *bad, int ntq)
 {
     __shared__ __align__(16) AttnLds<HD> L;  // 79 KB at HD = 256
-    if (bad && !attn_bad(bad, ntq)) return;  // k_attn_pairs has taken it
+    if (bad && !attn_bad(bad, ntq)) return;  // k_attn_split has taken it
     constexpr int NS = HD / 4, NC = HD / 16;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, c = lane & 15;
     const int q0 = blockIdx.x * 64 + 16 * wave;
@@ -341,21 +343,22 @@ __global__ void k_attn_merge(float *out, const float *Op, const float *mlp, int 
 }
 
 // ---------------------------------------------------------------------------
-// The same attention with fp16 operand pairs (v_mfma_f32_32x32x16_f16), for
-// the sequences whose products, and not their launches, take the time.
+// The same attention with every operand split into three bf16 parts
+// (v_mfma_f32_32x32x16_bf16), for the sequences whose products, and not their
+// launches, take the time.
 //
-// Every operand is x * s = hi + lo, s a power of two per row of Q and of K and
-// per column of V (|x * s| < 2^14; 2^13 for the softmax weights), hi and
-// lo each rounded to nearest, so hi + lo holds x to 2^-24 of itself or, where
-// fp16 has no smaller step, to 2^-38 of the largest value of its row or column;
-// a product is hi*hi + hi*lo + lo*hi, what is dropped is below 2^-24 of it, and
-// the sums are fp32: the rounding of fp32 products at 3/16 of their matrix
-// time.  The pairs are made once per call (k_attn_prep), not once per work
-// group.
-// Operands that hold a NaN, an infinity or a value past 2^60 take k_attn_mma
-// instead, decided on the device (bad[]): below that the product of two rows'
-// scales is far from overflow, so a score of 0 stays 0 and every score that
-// is finite in fp32 stays finite.
+// x = x1 + x2 + x3, each part the rest rounded to nearest: 3 x 8 significant
+// bits hold all 24 of x, and bf16 has fp32's exponents, so the parts need no
+// scale and a value loses nothing beside a larger one of its row or column.  A
+// product is x1*y1 + x1*y2 + x2*y1 + x2*y2 + x1*y3 + x3*y1; what is dropped is
+// below 2^-23 of it, of the order of an fp32 product's own rounding, and the
+// sums are fp32: 6/16 of the matrix time of fp32 products.  Q, K and V are
+// split once per call (k_attn_prep), the softmax weights, times 2^24 so that
+// the smallest have all their parts too, in the kernel.
+// Operands that hold a NaN, an infinity, a value past 2^59 (whose partial
+// products could overflow where the fp32 sum does not) or a non-zero one below
+// 2^-100 (whose last part would be subnormal) take k_attn_mma instead, decided
+// on the device (bad[]).
 //
 // Work group: 4 waves of 32 query rows each and one split of the keys, tiles
 // of 32 keys.  Scores are formed transposed, S^T = K Q^T, so that a lane holds
@@ -363,60 +366,43 @@ __global__ void k_attn_merge(float *out, const float *Op, const float *mlp, int 
 // exchange between the lane halves, and the weights are already in the B
 // layout of O^T = V^T P^T once V^T's keys are stored in that order (key
 // position 8h + e of a step of 16 is key 4h + e for e < 4, 8 + 4h + e - 4
-// beyond).  A tile of K and V (64 KB at HD = 256) goes from memory straight
-// into LDS while the one before is used, one barrier per tile.
+// beyond).  K and V of a tile (48 KB each at HD = 256) go from memory straight
+// into one LDS slot each: V's while the scores are formed, the next K's during
+// the products with V.
 //
-// What bounds it: Q's pairs and O take 256 registers at HD = 256, so a SIMD
-// holds one wave, and its matrix, exponential and LDS phases follow each
-// other: the matrix cores are 31 % busy (4096 x 256: 83 us of 110 for the
-// call; with k_attn_mma 254).  Error against 64 bits there 4e-7 (fp32: 7e-7).
+// What bounds it: Q's parts and O take 320 registers at HD = 256, so a SIMD
+// holds one wave, whose matrix, exponential and LDS phases follow each other:
+// the matrix cores are 39 % busy, beside 760 other vector instructions per
+// wave and tile (4096 x 256: 116 us of 132 for the call; k_attn_mma takes 254).
+// Operand reads two steps ahead instead of one, and two accumulators in turn,
+// measured the same.  Error against 64 bits there 4.1e-7 (k_attn_mma 7.0e-7).
+// Two fp16 halves per operand, scaled by row and column, take half the
+// products and 107 us, but lose what lies 2^-38 below its row's or column's
+// largest value, where it may be all that counts.
 // ---------------------------------------------------------------------------
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef __bf16 v8b __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 constexpr int AS_TK = 32, AS_ROWS = 128;  // keys per tile, query rows per work group
-constexpr float AS_MAX = 0x1p60f;           // largest operand the pairs take
+constexpr float AS_MAX = 0x1p59f, AS_MIN = 0x1p-100f;  // magnitudes that are split
 
 struct AttnPrep {
-    _Float16 *q;      // [rows][hi, lo][HD]
-    uint4 *kv;        // per tile [K hi][K lo] 32 x HD, [V hi][V lo] HD x 32
-    float *qinv, *kinv, *vinv;
-    int *bad;         // [tiles][Q, K, V]: not all of the tile's values are within AS_MAX
+    __bf16 *q;        // [rows][part][HD]
+    uint4 *kv;        // per tile [K part] 32 x HD, [V part] HD x 32
+    int *bad;         // [tiles][Q, K, V]: not all of the tile's values are to be split
 };
 
-// Column maxima of V over a slice of rows: part[blockIdx.x][HD] (hd % 4 == 0).
-constexpr int AS_PARTS = 32;
-
-__global__ void __launch_bounds__(256) k_attn_colmax(float *part, const float *V, int seq, int hd,
-                                                     int HD)
+__device__ __forceinline__ bool attn_splits_exactly(float x)
 {
-    const int per = (seq + AS_PARTS - 1) / AS_PARTS;
-    const int lo = blockIdx.x * per, hi = min(seq, lo + per);
-    const int nc = HD / 4, c = 4 * (threadIdx.x % nc), rstep = 256 / nc;
-    __shared__ __align__(16) v4f red[256];
-    v4f m = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (c < hd) {
-#pragma unroll 16
-        for (int r = lo + threadIdx.x / nc; r < hi; r += rstep) {
-            const v4f v = *reinterpret_cast<const v4f *>(V + (size_t)r * hd + c);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) m[e] = fmaxf(m[e], fabsf(v[e]));
-        }
-    }
-    red[threadIdx.x] = m;
-    __syncthreads();
-    if ((int)threadIdx.x >= nc) return;
-    for (int i = 1; i < rstep; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) m[e] = fmaxf(m[e], red[threadIdx.x + i * nc][e]);
-    *reinterpret_cast<v4f *>(part + (size_t)blockIdx.x * HD + c) = m;
+    const float a = fabsf(x);
+    return a == 0.0f || (a >= AS_MIN && a <= AS_MAX);
 }
 
-__device__ __forceinline__ float attn_scale(float amax)  // power of two, amax * s in [2^13, 2^14)
+__device__ __forceinline__ void split3(float x, __bf16 &a, __bf16 &b, __bf16 &c)
 {
-    if (!(amax > 0.0f) || !(amax <= 3.0e38f)) return 1.0f;
-    int e = 13 - ilogbf(amax);
-    e = e < -126 ? -126 : (e > 126 ? 126 : e);
-    return ldexpf(1.0f, e);
+    a = (__bf16)x;
+    const float r = x - (float)a;
+    b = (__bf16)r;
+    c = (__bf16)(r - (float)b);
 }
 
 // The 16-byte chunk j of a row of K lies at position j ^ attn_kswz(row), so that
@@ -428,15 +414,14 @@ __device__ __forceinline__ int attn_kswz(int r)
 }
 
 template <int HD>
-__global__ void __launch_bounds__(256) k_attn_prep(AttnPrep P, const float *part, const float *Q,
-                                                   const float *K, const float *V, int seq, int hd,
-                                                   int nt)
+__global__ void __launch_bounds__(256) k_attn_prep(AttnPrep P, const float *Q, const float *K,
+                                                   const float *V, int seq, int hd, int nt)
 {
     constexpr int W = HD / 64;  // columns per lane of a row
     // blockIdx.y: Q, K or V of tile blockIdx.x
     const int t = blockIdx.x, which = blockIdx.y;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    _Float16 *kt = reinterpret_cast<_Float16 *>(P.kv) + (size_t)t * 4 * AS_TK * HD;
+    __bf16 *kt = reinterpret_cast<__bf16 *>(P.kv) + (size_t)t * 6 * AS_TK * HD;
     bool ok = true;
     if (which && t >= nt) {
         // past the last tile of keys: nothing to write but the flag
@@ -456,31 +441,20 @@ __global__ void __launch_bounds__(256) k_attn_prep(AttnPrep P, const float *part
 #pragma unroll
         for (int i = 0; i < NR; ++i) {
             const int lr = wave * NR + i, r = t * AS_TK + lr;
-            float m = 0.0f;
+            __bf16 part[3][W];
 #pragma unroll
             for (int j = 0; j < W; ++j) {
-                ok = ok && fabsf(x[i][j]) <= AS_MAX;
-                m = fmaxf(m, fabsf(x[i][j]));
+                ok = ok && attn_splits_exactly(x[i][j]);
+                split3(x[i][j], part[0][j], part[1][j], part[2][j]);
             }
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-            const float s = attn_scale(m);
-            _Float16 *dh = which ? kt + (size_t)lr * HD : P.q + (size_t)r * 2 * HD;
-            _Float16 *dl = which ? dh + AS_TK * HD : dh + HD;
-            _Float16 hi[W], lo[W];
-#pragma unroll
-            for (int j = 0; j < W; ++j) {
-                const float v = x[i][j] * s;
-                hi[j] = (_Float16)v;
-                lo[j] = (_Float16)(v - (float)hi[j]);
-            }
+            __bf16 *d = which ? kt + (size_t)lr * HD : P.q + (size_t)r * 3 * HD;
             const int o = which ? 8 * ((W * lane / 8) ^ attn_kswz<HD>(lr)) + W * lane % 8 : W * lane;
-            __builtin_memcpy(__builtin_assume_aligned(dh + o, 2 * W), hi, 2 * W);
-            __builtin_memcpy(__builtin_assume_aligned(dl + o, 2 * W), lo, 2 * W);
-            if (lane == 0) (which ? P.kinv : P.qinv)[r] = 1.0f / s;
+#pragma unroll
+            for (int n = 0; n < 3; ++n)
+                __builtin_memcpy(__builtin_assume_aligned(d + n * (which ? AS_TK * HD : HD) + o, 2 * W),
+                                 part[n], 2 * W);
         }
     } else {
-        __shared__ float vs[HD];
         constexpr int NV = 4 * HD / 256;  // runs of 8 keys of one column per thread
         float x[NV][8];
 #pragma unroll
@@ -492,145 +466,141 @@ __global__ void __launch_bounds__(256) k_attn_prep(AttnPrep P, const float *part
                 x[n][e] = r < seq && c < hd ? V[(size_t)r * hd + c] : 0.0f;
             }
         }
-        if (tid < HD) {
-            float m = 0.0f;
-#pragma unroll
-            for (int i = 0; i < AS_PARTS; ++i) m = fmaxf(m, part[(size_t)i * HD + tid]);
-            const float s = attn_scale(m);
-            vs[tid] = s;
-            if (t == 0) P.vinv[tid] = 1.0f / s;
-        }
-        __syncthreads();
-        _Float16 *vt = kt + 2 * AS_TK * HD;
+        __bf16 *vt = kt + 3 * AS_TK * HD;
 #pragma unroll
         for (int n = 0; n < NV; ++n) {
             const int i = tid + 256 * n, c = i % HD, ch = i / HD;
-            v8h hi, lo;
+            v8b part[3];
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                ok = ok && fabsf(x[n][e]) <= AS_MAX;
-                const float v = x[n][e] * vs[c];
-                hi[e] = (_Float16)v;
-                lo[e] = (_Float16)(v - (float)hi[e]);
+                __bf16 p0, p1, p2;
+                ok = ok && attn_splits_exactly(x[n][e]);
+                split3(x[n][e], p0, p1, p2);
+                part[0][e] = p0;
+                part[1][e] = p1;
+                part[2][e] = p2;
             }
             // a column's four 16-byte chunks are rotated among themselves by
             // its number, so that 16 lanes' reads cover every LDS bank
             const int o = c * AS_TK + 8 * (ch ^ ((c >> 2) & 3));
-            *reinterpret_cast<v8h *>(vt + o) = hi;
-            *reinterpret_cast<v8h *>(vt + AS_TK * HD + o) = lo;
+#pragma unroll
+            for (int m = 0; m < 3; ++m) *reinterpret_cast<v8b *>(vt + m * AS_TK * HD + o) = part[m];
         }
     }
     const int any = __syncthreads_or(!ok);
     if (tid == 0) P.bad[3 * t + which] = any;
 }
 
-// 16 bytes per lane from global memory into LDS at base + 16 * lane, base the
-// same in every lane; complete after the wave's next wait for its loads.  (As
-// asm: for the builtin the compiler waits for the load before any LDS read.)
+// 16 bytes per lane from g + off (g the same in every lane) into LDS at base +
+// 16 * lane; complete after the wave's next wait for its loads.  (As asm: for
+// the builtin the compiler waits for the load before any LDS read.)
 __device__ __forceinline__ uint32_t lds_addr(const void *p)
 {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char *)p;
 }
-__device__ __forceinline__ void lds_load16(const void *g, uint32_t base)
+__device__ __forceinline__ void lds_load16(const void *g, uint32_t off, uint32_t base)
 {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                  :
-                 : "s"(__builtin_amdgcn_readfirstlane(base)), "v"(g)
+                 : "s"(__builtin_amdgcn_readfirstlane(base)), "v"(off), "s"(g)
                  : "memory", "m0");
 }
 
 // Keeps a value in the accumulator half of the register file, which the matrix
-// instructions read and write directly: O and Q take it all, and left to
-// itself the compiler moves O across the halves in every tile.
+// instructions read and write directly: O and most of Q take it all, and left
+// to itself the compiler moves O across the halves in every tile.
 template <class T>
 __device__ __forceinline__ void agpr(T &v)
 {
     asm volatile("" : "+a"(v));
 }
 
+__device__ __forceinline__ v16f mfma_bf16(v8b a, v8b b, v16f c)
+{
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
 template <int HD>
-struct AttnSplitLds {  // one tile's image per slot
-    _Float16 k[2][2][AS_TK * HD];  // [slot][hi, lo]
-    _Float16 v[2][2][HD * AS_TK];
-    float kinv[2][AS_TK], vinv[HD];
+struct AttnSplitLds {  // one tile's image
+    __bf16 k[3][AS_TK * HD];
+    __bf16 v[3][HD * AS_TK];
 };
 
 template <int HD>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
-    k_attn_pairs(float *out, float *Op, float *mlp, AttnPrep P, int seq, int hd, float scale,
+    k_attn_split(float *out, float *Op, float *mlp, AttnPrep P, int seq, int hd, float scale,
                  int nt, int ntq, int tiles_per_split)
 {
     __shared__ __align__(16) AttnSplitLds<HD> L;
-    constexpr int NK = HD / 16, NJ = HD / 32, NL = HD / 32;  // NL: 16-byte words per thread of K, of V
+    constexpr int NK = HD / 16, NJ = HD / 32, NL = 3 * HD / 64;  // NL: 16-byte words per thread of K, of V
     if (attn_bad(P.bad, ntq)) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane & 31, h = lane >> 5;
     const int row = blockIdx.y * AS_ROWS + 32 * wave + q;
     const int t_lo = blockIdx.x * tiles_per_split, t_hi = min(nt, t_lo + tiles_per_split);
 
-    v8h qh[NK], ql[NK];
+    v8b qv[3][NK];
     {
-        const _Float16 *qr = P.q + (size_t)row * 2 * HD + 8 * h;
+        const __bf16 *qr = P.q + (size_t)row * 3 * HD + 8 * h;
+#pragma unroll
+        for (int n = 0; n < 3; ++n)
+#pragma unroll
+            for (int s = 0; s < NK; ++s)
+                qv[n][s] = *reinterpret_cast<const v8b *>(qr + n * HD + 16 * s);
 #pragma unroll
         for (int s = 0; s < NK; ++s) {
-            qh[s] = *reinterpret_cast<const v8h *>(qr + 16 * s);
-            ql[s] = *reinterpret_cast<const v8h *>(qr + HD + 16 * s);
-        }
-#pragma unroll
-        for (int s = 0; s < NK; ++s) {
-            agpr(qh[s]);
-            agpr(ql[s]);
+            agpr(qv[0][s]);
+            agpr(qv[1][s]);
         }
     }
-    const float qs = P.qinv[row] * scale;
 
-    // K or V of one tile straight into LDS: 1 KB per wave and load.  Tiles
-    // past the split re-read its last one, unused.
-    auto load = [&](int t, int slot) {
-        const uint4 *p = P.kv + (size_t)min(t, t_hi - 1) * (16 * HD) + 64 * wave + lane;
-        const uint32_t k = lds_addr(&L.k[slot][0][0]) + 1024 * wave;
-        const uint32_t v = lds_addr(&L.v[slot][0][0]) + 1024 * wave;
+    // K or V of a tile straight into LDS: 1 KB per wave and load
+    auto load = [&](const uint4 *p, const void *dst) {
+        const uint32_t d = lds_addr(dst) + 1024 * wave;
 #pragma unroll
-        for (int i = 0; i < NL; ++i) lds_load16(p + 256 * i, k + 4096 * i);
-#pragma unroll
-        for (int i = 0; i < NL; ++i) lds_load16(p + 8 * HD + 256 * i, v + 4096 * i);
+        for (int i = 0; i < NL; ++i) lds_load16(p + 256 * i, 16 * tid, d + 4096 * i);
     };
-    // S^T of one tile: this lane's query, keys 8 (r / 4) + 4h + r % 4
-    // (two steps' operands are read while the two before them multiply)
-    auto scores = [&](int slot) {
-        v16f s0 = {}, s1 = {};
-        v8h kb[2][2][2];
-        auto read = [&](v8h(&r)[2][2], int s2) {
+    auto load_k = [&](int t) { load(P.kv + (size_t)t * (24 * HD), &L.k[0][0]); };
+    auto load_v = [&](int t) { load(P.kv + (size_t)t * (24 * HD) + 12 * HD, &L.v[0][0]); };
+    // This wave's loads have arrived; past the barrier every wave's have, and
+    // every wave is done with what it read before it.
+    auto arrived = [&] {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    };
+    // S^T of one tile: this lane's query, keys 8 (r / 4) + 4h + r % 4 (a
+    // step's operands are read while the step before it multiplies)
+    auto scores = [&] {
+        v16f s0 = {}, s1 = {};  // the products of the first parts; the others
+        v8b kb[2][3];
+        auto read = [&](v8b(&r)[3], int s) {
+            const int off = q * HD + 8 * ((2 * s + h) ^ attn_kswz<HD>(q));
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int off = q * HD + 8 * ((2 * (s2 + i) + h) ^ attn_kswz<HD>(q));
-                r[i][0] = *reinterpret_cast<const v8h *>(&L.k[slot][0][off]);
-                r[i][1] = *reinterpret_cast<const v8h *>(&L.k[slot][1][off]);
-            }
+            for (int n = 0; n < 3; ++n) r[n] = *reinterpret_cast<const v8b *>(&L.k[n][off]);
         };
         read(kb[0], 0);
 #pragma unroll
-        for (int s = 0; s < NK; s += 2) {
-            if (s + 2 < NK) read(kb[(s / 2 + 1) & 1], s + 2);
+        for (int s = 0; s < NK; ++s) {
+            if (s + 1 < NK) read(kb[(s + 1) & 1], s + 1);
             __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const v8h kh = kb[(s / 2) & 1][i][0], kl = kb[(s / 2) & 1][i][1];
-                s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, qh[s + i], s0, 0, 0, 0);
-                s1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, ql[s + i], s1, 0, 0, 0);
-                s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl, qh[s + i], s0, 0, 0, 0);
-            }
+            const v8b(&k)[3] = kb[s & 1];
+            s1 = mfma_bf16(k[2], qv[0][s], s1);
+            s0 = mfma_bf16(k[0], qv[0][s], s0);
+            s1 = mfma_bf16(k[0], qv[2][s], s1);
+            s1 = mfma_bf16(k[1], qv[1][s], s1);
+            s1 = mfma_bf16(k[1], qv[0][s], s1);
+            s1 = mfma_bf16(k[0], qv[1][s], s1);
             __builtin_amdgcn_sched_barrier(0);
         }
         return s0 + s1;
     };
 
-    auto read_v = [&](v8h(&r)[2][2], int slot, int j) {
+    auto read_v = [&](v8b(&r)[2][3], int j) {
         const int c = 32 * j + q;
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             const int off = c * AS_TK + 8 * ((2 * s + h) ^ ((c >> 2) & 3));
-            r[s][0] = *reinterpret_cast<const v8h *>(&L.v[slot][0][off]);
-            r[s][1] = *reinterpret_cast<const v8h *>(&L.v[slot][1][off]);
+#pragma unroll
+            for (int n = 0; n < 3; ++n) r[s][n] = *reinterpret_cast<const v8b *>(&L.v[n][off]);
         }
     };
 
@@ -642,38 +612,22 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     }
     float m = -INFINITY, l = 0.0f;
 
-    if (tid < HD) L.vinv[tid] = P.vinv[tid];
-    float rki = P.kinv[min(t_lo + 1, t_hi - 1) * AS_TK + (tid & (AS_TK - 1))];  // of tile t + 1
-    if (tid < AS_TK) L.kinv[0][tid] = P.kinv[t_lo * AS_TK + tid];
-    load(t_lo, 0);
+    load_k(t_lo);
     for (int t = t_lo; t < t_hi; ++t) {
-        const int cur = (t - t_lo) & 1, nxt = cur ^ 1;
 #pragma unroll
         for (int j = 0; j < NJ; ++j) agpr(o[j]);
-        // Tile t has arrived, and every wave is past tile t - 1, whose slot
-        // takes t + 1.
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        asm volatile("" : "+v"(rki));
-        __syncthreads();
-        if (tid < AS_TK) L.kinv[nxt][tid] = rki;
-        rki = P.kinv[min(t + 2, t_hi - 1) * AS_TK + (tid & (AS_TK - 1))];
-        load(t + 1, nxt);
+        arrived();  // K of tile t; V of tile t - 1 is consumed
+        load_v(t);
         __builtin_amdgcn_sched_barrier(0);
-        const v16f sc = scores(cur);
-        v8h vb[2][2][2];
-        read_v(vb[0], cur, 0);
+        const v16f sc = scores();
         __builtin_amdgcn_sched_barrier(0);
         float p[16];
         float tm = -INFINITY;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const v4f ki = *reinterpret_cast<const v4f *>(&L.kinv[cur][8 * i + 4 * h]);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float v = sc[4 * i + e] * (ki[e] * qs);
-                p[4 * i + e] = AS_TK * t + 8 * i + 4 * h + e < seq ? v : -INFINITY;
-                tm = fmaxf(tm, p[4 * i + e]);
-            }
+        for (int i = 0; i < 16; ++i) {
+            const float v = sc[i] * scale;
+            p[i] = AS_TK * t + 8 * (i >> 2) + 4 * h + (i & 3) < seq ? v : -INFINITY;
+            tm = fmaxf(tm, p[i]);
         }
         tm = fmaxf(tm, __shfl_xor(tm, 32, 64));
         // The reference m moves only when the maximum has grown past it by a
@@ -685,6 +639,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
             l *= corr;
 #pragma unroll
             for (int j = 0; j < NJ; ++j) {
+                agpr(o[j]);  // 16 of O at a time in the other half
+                __builtin_amdgcn_sched_barrier(0);
                 v16f x = o[j] * corr;
                 agpr(x);
                 o[j] = x;
@@ -698,25 +654,34 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
             l += p[r];
         }
         m = mn;
-        v8h ph[2], pl[2];
+        v8b pv[2][3];
 #pragma unroll
         for (int s = 0; s < 2; ++s)
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const float v = p[8 * s + e] * 8192.0f;
-                ph[s][e] = (_Float16)v;
-                pl[s][e] = (_Float16)(v - (float)ph[s][e]);
+                __bf16 p0, p1, p2;
+                split3(p[8 * s + e] * 0x1p24f, p0, p1, p2);
+                pv[s][0][e] = p0;
+                pv[s][1][e] = p1;
+                pv[s][2][e] = p2;
             }
+        arrived();  // V of tile t; its K is consumed
+        if (t + 1 < t_hi) load_k(t + 1);
+        v8b vb[2][2][3];
+        read_v(vb[0], 0);
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            if (j + 1 < NJ) read_v(vb[(j + 1) & 1], cur, j + 1);
+            if (j + 1 < NJ) read_v(vb[(j + 1) & 1], j + 1);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
-                const v8h vh = vb[j & 1][s][0], vl = vb[j & 1][s][1];
-                o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, ph[s], o[j], 0, 0, 0);
-                o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, pl[s], o[j], 0, 0, 0);
-                o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl, ph[s], o[j], 0, 0, 0);
+                const v8b(&v)[3] = vb[j & 1][s];
+                o[j] = mfma_bf16(v[2], pv[s][0], o[j]);
+                o[j] = mfma_bf16(v[0], pv[s][2], o[j]);
+                o[j] = mfma_bf16(v[1], pv[s][1], o[j]);
+                o[j] = mfma_bf16(v[1], pv[s][0], o[j]);
+                o[j] = mfma_bf16(v[0], pv[s][1], o[j]);
+                o[j] = mfma_bf16(v[0], pv[s][0], o[j]);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -724,7 +689,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     l += __shfl_xor(l, 32, 64);
     if (row >= seq) return;
     const int nsplit = gridDim.x;
-    float f = 1.0f / 8192.0f;
+    float f = 0x1p-24f;
     float *po;
     if (nsplit == 1) {
         const float em = expf(m);
@@ -743,10 +708,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
         for (int i = 0; i < 4; ++i) {
             const int c = 32 * j + 8 * i + 4 * h;
             if (c >= hd) continue;  // hd % 4 == 0
-            const v4f vi = *reinterpret_cast<const v4f *>(&L.vinv[c]);
             v4f r;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) r[e] = o[j][4 * i + e] * f * vi[e];
+            for (int e = 0; e < 4; ++e) r[e] = o[j][4 * i + e] * f;
             *reinterpret_cast<v4f *>(po + c) = r;
         }
 }
@@ -822,17 +786,18 @@ static int attn_splits(int seq)
 
 static int attn_hd(int hd) { return hd <= 64 ? 64 : hd <= 128 ? 128 : 256; }
 
-// Pairs (k_attn_pairs) from where their three more launches are paid back;
-// fp32 / pairs, us per call: hd = 256 1400 keys 67 / 65, 1700 77 / 66, 4096
-// 254 / 110; hd = 128 1400 54 / 57, 1700 58 / 57, 4096 154 / 82; hd = 64 1700
-// 44 / 48, 2048 49 / 50, 3000 70 / 58.
-static int attn_pairs(int seq, int hd)
+// Parts (k_attn_split) from where their two more launches are paid back at
+// every head dim; fp32 / parts, us per call: hd = 256 1152 keys 62 / 59, 1408
+// 68 / 63, 1700 78 / 66, 4096 258 / 138; hd = 128 1152 50 / 49, 1408 55 / 54,
+// 1536 57 / 52, 4096 154 / 93; hd = 64 1600 43 / 43, 1792 45 / 43, 2176 52 /
+// 47, 4096 99 / 69.
+static int attn_split(int seq, int hd)
 {
     const int HD = attn_hd(hd);
-    return seq >= (HD == 256 ? 1536 : HD == 128 ? 1700 : 2176);
+    return seq >= (HD == 64 ? 1792 : 1536);
 }
 
-static int attn_pair_splits(int seq, int *per)
+static int attn_key_splits(int seq, int *per)
 {
     const int nq = (seq + AS_ROWS - 1) / AS_ROWS, nt = (seq + AS_TK - 1) / AS_TK;
     int ns = 256 / nq;
@@ -842,7 +807,7 @@ static int attn_pair_splits(int seq, int *per)
 }
 
 struct AttnWs {
-    size_t q, kv, qinv, kinv, vinv, bad, part, op, ml, bytes;
+    size_t q, kv, bad, op, ml, bytes;
 };
 
 static AttnWs attn_ws(int seq, int hd)
@@ -850,7 +815,7 @@ static AttnWs attn_ws(int seq, int hd)
     const int HD = attn_hd(hd), rq = (seq + AS_ROWS - 1) / AS_ROWS * AS_ROWS;
     const int rk = (seq + AS_TK - 1) / AS_TK * AS_TK;
     int per;
-    const int ns = attn_pair_splits(seq, &per);
+    const int ns = attn_key_splits(seq, &per);
     AttnWs w;
     size_t off = 0;
     auto take = [&](size_t n) {
@@ -858,13 +823,9 @@ static AttnWs attn_ws(int seq, int hd)
         off += (n + 255) & ~(size_t)255;
         return o;
     };
-    w.q = take((size_t)rq * HD * 4);
-    w.kv = take((size_t)rk * HD * 8);
-    w.qinv = take((size_t)rq * 4);
-    w.kinv = take((size_t)rk * 4);
-    w.vinv = take((size_t)HD * 4);
+    w.q = take((size_t)rq * HD * 6);
+    w.kv = take((size_t)rk * HD * 12);
     w.bad = take((size_t)(rq / AS_TK) * 12);
-    w.part = take((size_t)AS_PARTS * HD * 4);
     w.op = take(ns > 1 ? (size_t)ns * seq * hd * 4 : 0);
     w.ml = take(ns > 1 ? (size_t)ns * seq * 8 : 0);
     w.bytes = off;
@@ -873,7 +834,7 @@ static AttnWs attn_ws(int seq, int hd)
 
 extern "C" size_t ornk_attention_mma_ws(int seq, int hd)
 {
-    if (attn_pairs(seq, hd)) return attn_ws(seq, hd).bytes;
+    if (attn_split(seq, hd)) return attn_ws(seq, hd).bytes;
     const int ns = attn_splits(seq);
     return ns > 1 ? (size_t)ns * seq * (hd + 2) * sizeof(float) : 0;
 }
@@ -887,26 +848,21 @@ static void attn_merge(float *out, const float *Op, const float *mlp, int seq, i
 }
 
 template <int HD>
-static void attn_pairs_launch(float *out, const float *Q, const float *K, const float *V, int seq,
+static void attn_split_launch(float *out, const float *Q, const float *K, const float *V, int seq,
                               int hd, float scale, uint8_t *ws, hipStream_t s)
 {
     const AttnWs w = attn_ws(seq, hd);
     const int nq = (seq + AS_ROWS - 1) / AS_ROWS, nt = (seq + AS_TK - 1) / AS_TK;
     const int ntq = nq * (AS_ROWS / AS_TK);
     int per;
-    const int ns = attn_pair_splits(seq, &per);
+    const int ns = attn_key_splits(seq, &per);
     AttnPrep P;
-    P.q = reinterpret_cast<_Float16 *>(ws + w.q);
+    P.q = reinterpret_cast<__bf16 *>(ws + w.q);
     P.kv = reinterpret_cast<uint4 *>(ws + w.kv);
-    P.qinv = reinterpret_cast<float *>(ws + w.qinv);
-    P.kinv = reinterpret_cast<float *>(ws + w.kinv);
-    P.vinv = reinterpret_cast<float *>(ws + w.vinv);
     P.bad = reinterpret_cast<int *>(ws + w.bad);
-    float *part = reinterpret_cast<float *>(ws + w.part);
     float *Op = reinterpret_cast<float *>(ws + w.op), *mlp = reinterpret_cast<float *>(ws + w.ml);
-    hipLaunchKernelGGL(k_attn_colmax, dim3(AS_PARTS), dim3(256), 0, s, part, V, seq, hd, HD);
-    hipLaunchKernelGGL(k_attn_prep<HD>, dim3(ntq, 3), dim3(256), 0, s, P, part, Q, K, V, seq, hd, nt);
-    hipLaunchKernelGGL(k_attn_pairs<HD>, dim3(ns, nq), dim3(256), 0, s, out, Op, mlp, P, seq, hd,
+    hipLaunchKernelGGL(k_attn_prep<HD>, dim3(ntq, 3), dim3(256), 0, s, P, Q, K, V, seq, hd, nt);
+    hipLaunchKernelGGL(k_attn_split<HD>, dim3(ns, nq), dim3(256), 0, s, out, Op, mlp, P, seq, hd,
                        scale, nt, ntq, per);
     // the same splits (twice as many tiles of half the keys), the same partials
     hipLaunchKernelGGL(k_attn_mma<HD>, dim3((seq + 63) / 64, ns), dim3(256), 0, s, out, Op, mlp, Q, K,
@@ -919,12 +875,12 @@ extern "C" int ornk_attention_mma(float *out, const float *Q, const float *K, co
 {
     if (seq <= 0 || hd <= 0) return hipSuccess;
     if (hd % 4 || hd > 256) return hipErrorInvalidValue;
-    if (attn_pairs(seq, hd)) {
+    if (attn_split(seq, hd)) {
         if (!ws) return hipErrorInvalidValue;
         uint8_t *w = static_cast<uint8_t *>(ws);
-        if (hd <= 64) attn_pairs_launch<64>(out, Q, K, V, seq, hd, scale, w, s);
-        else if (hd <= 128) attn_pairs_launch<128>(out, Q, K, V, seq, hd, scale, w, s);
-        else attn_pairs_launch<256>(out, Q, K, V, seq, hd, scale, w, s);
+        if (hd <= 64) attn_split_launch<64>(out, Q, K, V, seq, hd, scale, w, s);
+        else if (hd <= 128) attn_split_launch<128>(out, Q, K, V, seq, hd, scale, w, s);
+        else attn_split_launch<256>(out, Q, K, V, seq, hd, scale, w, s);
         return hipGetLastError();
     }
     const int nt = (seq + AM_TK - 1) / AM_TK;

@@ -186,9 +186,9 @@ def run_attention(om, ctx, Q, K, V, in_place=False):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("seq,hd", [(1536, 256), (1541, 252), (1700, 128), (1763, 96), (2176, 64),
-                                    (2209, 60), (4129, 256)])
+                                    (2209, 60), (4129, 256), (1536, 128), (1792, 64)])
 def test_gpu_attention_pairs(om, ctx, seq, hd):
-    """Sequences long enough for the fp16-pair kernel, at and past its tiles
+    """Sequences long enough for the kernel on bf16 parts, at and past its tiles
     of 32 keys and 128 rows and its padded head dims.  Columns of V, rows of
     Q and of K have scales far apart (a power of two each, taken out of the
     other operand, so that the scores stay the plain ones'): within 2e-6 of
@@ -223,8 +223,8 @@ def test_gpu_attention_pairs_growing_and_large_scores(om, ctx):
 
 @pytest.mark.gpu
 def test_gpu_attention_pairs_not_finite(om, ctx):
-    """An infinity or NaN stays where fp32 arithmetic puts it: the pair
-    kernel leaves such operands to the fp32 one."""
+    """An infinity or NaN stays where fp32 arithmetic puts it: the kernel on
+    bf16 parts leaves such operands to the fp32 one."""
     rng = np.random.default_rng(4)
     seq, hd = 2180, 64
     Q, K, V = (f32(rng.standard_normal((seq, hd))) for _ in range(3))
@@ -244,9 +244,10 @@ def test_gpu_attention_pairs_not_finite(om, ctx):
 @pytest.mark.parametrize("big,small", [(1e30, 1.0), (2.0 ** 60, 2.0 ** -60), (2.0 ** 61, 2.0 ** -61)])
 def test_gpu_attention_pairs_huge_operands(om, ctx, big, small):
     """Rows of Q and K with huge values in columns that the other one leaves
-    at 0: the scores are the rest's, at any magnitude that fp32 holds (the
-    product of the rows' own scales would not be one).  Tolerance as for the
-    plain scores, whose products and sums these are."""
+    at 0, past the magnitudes that are split into parts (2^59): the scores are
+    the rest's, at any magnitude that fp32 holds.  What lies beside the large
+    values is 0 or so small that every score is about 0, so this shows overflow
+    and not the loss of small values (test_gpu_attention_wide_range_scores)."""
     rng = np.random.default_rng(5)
     seq, hd = 2180, 64
     Q, K, V = (f32(rng.standard_normal((seq, hd))) for _ in range(3))
@@ -255,6 +256,62 @@ def test_gpu_attention_pairs_huge_operands(om, ctx, big, small):
     Q[:, 2:], K[:, 2:] = (0, 0) if small == 1.0 else (Q[:, 2:] * small, K[:, 2:] * small)
     ref = attention64(Q, K, V)
     assert np.abs(run_attention(om, ctx, Q, K, V) - ref).max() < 2e-6 * np.abs(ref).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("seq,hd", [(2180, 64), (1700, 128), (1540, 256), (2190, 4), (2200, 12)])
+@pytest.mark.parametrize("b", [0, 16, 20, 24, 30, 40, 50, 58])
+def test_gpu_attention_wide_range_scores(om, ctx, seq, hd, b):
+    """Columns of Q and of K that are 2^b where the other operand is 0: the
+    scores are the other columns', standard normal, and nothing of those may
+    be lost beside the large ones.  The plain scores' 2e-6."""
+    rng = np.random.default_rng(b + hd)
+    Q, K, V = (f32(rng.standard_normal((seq, hd))) for _ in range(3))
+    Q[:, 0], K[:, 0] = 2.0 ** b, 0
+    Q[:, 1], K[:, 1] = 0, 2.0 ** b
+    ref = attention64(Q, K, V)
+    err = np.abs(run_attention(om, ctx, Q, K, V) - ref).max() / np.abs(ref).max()
+    assert err < 2e-6, err
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b", [0, 16, 24, 30, 40, 50, 58, -20, -60, -90])
+@pytest.mark.parametrize("cols", [slice(None), slice(5, 6)])
+def test_gpu_attention_wide_range_values(om, ctx, b, cols):
+    """A value of 2^b, in one column or in all, at a key that no query attends
+    to (its score is 200 below the others'): 2e-6 in every column by itself."""
+    rng = np.random.default_rng(b + 100)
+    seq, hd = 2200, 64
+    Q, K, V = (f32(rng.standard_normal((seq, hd))) for _ in range(3))
+    Q[:, 0], K[:, 0] = 8, 0
+    K[7, 0] = -200
+    V[7, cols] = 2.0 ** b
+    if b < 0:  # and a key that every query attends to, with values as small
+        K[1200, 0] = 100
+        V[1200] = f32(rng.standard_normal(hd)) * f32(2.0 ** b)
+    ref = attention64(Q, K, V)
+    got = run_attention(om, ctx, Q, K, V)
+    err = (np.abs(got - ref).max(axis=0) / np.abs(ref).max(axis=0)).max()
+    assert err < 2e-6, err
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("gap", [10, 20, 40, 70])
+def test_gpu_attention_sink(om, ctx, gap):
+    """A key with value 0 takes all but e^-gap of every query's weight, so that
+    the outputs are made of weights that small.  Scores s of that size carry
+    fp32 rounding of up to |s| 2^-23 each, which the weights take over:
+    gap * 1.2e-7 beside the plain scores' 2e-6."""
+    rng = np.random.default_rng(gap)
+    seq, hd = 2200, 64
+    Q, K, V = (f32(rng.standard_normal((seq, hd))) for _ in range(3))
+    Q[:, 0], K[:, 0] = 8, 0
+    K[7] = 0
+    K[7, 0] = gap
+    V[7] = 0
+    ref = attention64(Q, K, V)
+    err = np.abs(run_attention(om, ctx, Q, K, V) - ref).max() / np.abs(ref).max()
+    assert err < 2e-6 + gap * 2.0 ** -23, err
 
 
 @pytest.mark.gpu
