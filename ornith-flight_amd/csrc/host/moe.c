@@ -936,7 +936,7 @@ int gpu_moe_store_get_experts(gpu_context *ctx, ornith_moe_store *st, int layer,
 
 typedef struct {
     int ks_gu, ks_dn, rows_max, items_max, tchunk;
-    int use_dec; /* MFMA path with the decode-shaped kernels (items <= 16 rows) */
+    int use_dec; /* MFMA path with the decode-shaped kernels (items <= 32 rows) */
     int use_blk; /* MFMA kernels on vec@mat blocks (items <= 32 rows) */
 } plan_t;
 
@@ -952,7 +952,7 @@ static int pow2_floor(int v)
  * into ks slices so the grid holds ~2048 blocks (8 per CU).  Slices keep at
  * least 32 rows (gate/up) and 32 rows (down) so the split-K partials stay a
  * small fraction of the weight bytes. */
-static plan_t make_plan(const ornith_moe_shape *sh, int T, int use_mfma)
+static plan_t make_plan(const ornith_moe_shape *sh, int T, int use_mfma, int most_rows)
 {
     plan_t p;
     memset(&p, 0, sizeof p);
@@ -960,17 +960,13 @@ static plan_t make_plan(const ornith_moe_shape *sh, int T, int use_mfma)
     const int D = sh->d_model, H = sh->hidden;
     /* MFMA work items hold at most one 16-row tile (the decode kernels) at
      * decode sizes, two (the decode kernels' two-tile instances) above 64
-     * tokens wherever the batch averages at most 32 rows per expert (16 below
-     * 192 tokens: fewer experts then, whose gate/up slices of 16 steps would
-     * take more partials than the fixed scratch holds), four (the prefill
-     * grouped GEMMs) beyond: with 256 experts and top 8 the layer takes
-     * 288 / 324 us (two tiles / four) at 600 tokens, 340 / 362 at 900,
-     * 369 / 381 at 1024, 389 / 391 at 1100, 497 / 425 at 1400.
+     * tokens wherever the batch averages at most `most_rows` rows per expert
+     * (16 or 32, choose_plan), four (the prefill grouped GEMMs) beyond.
      * Skewed batches (a few hot experts, many cold ones) then split each
      * hot expert into items of 32 rows instead of running every cold expert
      * through a 64-row tile: an item costs its weight conversion whatever
      * its rows. */
-    const int two = T * k <= (T >= 192 ? 32 : 16) * E; /* two tiles */
+    const int two = T * k <= most_rows * E; /* two tiles */
     p.tchunk = use_mfma ? (T <= 64 ? 16 : two ? 32 : 64) : (T <= 64 ? 2 : 8);
     p.rows_max = T * k + (sh->has_shared ? T : 0);
     const int max_slots = (T * k < E ? T * k : E) + (sh->has_shared ? 1 : 0);
@@ -1099,7 +1095,7 @@ static int make_plan_blk(const ornith_moe_shape *sh, int T, plan_t *out)
     while (D / 32 / kg > 64) kg *= 2;
     while (kg > 1 && ((D / 32) % kg || D / 32 / kg < 4)) kg /= 2;
     while (kd > 1 && ((H / 32) % kd || H / 32 / kd < 4 || kd > 16)) kd /= 2;
-    const plan_t v = make_plan(sh, T, 0);
+    const plan_t v = make_plan(sh, T, 0, 0);
     while (kg * 2 * H + kd * D > v.ks_gu * 2 * H + v.ks_dn * D) {
         const int g = kg > 1 && D / 32 / (kg / 2) <= 64, d = kd > 1 && H / 32 / (kd / 2) <= 64;
         if (g && (!d || kg * 2 * H >= kd * D)) kg /= 2;
@@ -1188,6 +1184,36 @@ static ws_t carve_ws(const ornith_moe_shape *sh, int T, const plan_t *p, int nor
     return w;
 }
 
+/* The plan of a forward (blocks: the kernels that read vec@mat blocks may
+ * run).  A plan that takes more work buffers than another of the same products
+ * gives way to it at sizes where only the other fits the fixed scratch, also in
+ * a call that may allocate (both give the same bits). */
+static plan_t choose_plan(const ornith_moe_shape *sh, int T, int use_mfma, int blocks, int norm,
+                          int cert)
+{
+#define FITS(p, amax) (carve_ws(sh, T, &(p), norm, cert, amax, ORNK_SYNC_BYTES).end <= ORNK_SCRATCH_BYTES)
+    if (sh->file_layout) return make_plan_file(sh, T);
+    plan_t p;
+    if (blocks && make_plan_blk(sh, T, &p)) {
+        /* its row maxima are a few bytes a row more than the VALU plan takes */
+        const plan_t v = make_plan(sh, T, 0, 0);
+        return !FITS(p, 1) && FITS(v, 0) ? v : p;
+    }
+    p = make_plan(sh, T, use_mfma, 32);
+    if (use_mfma && p.tchunk == 32 && T * sh->top_k > 16 * sh->n_experts) {
+        /* Between 16 and 32 rows per expert two-tile items are the faster (top
+         * 8, us with two tiles / four: 256 experts 288 / 324 at 600 tokens, 340
+         * / 362 at 900, 369 / 381 at 1024, and beyond 389 / 391 at 1100, 497 /
+         * 425 at 1400; 128 experts 147 / 179 at 260, 184 / 208 at 500; 64 experts
+         * 97 / 113 at 130, 121 / 133 at 250; 32 experts 78 / 91 at 70, 87 / 104
+         * at 128), but their slices can take more partials */
+        const plan_t v = make_plan(sh, T, use_mfma, 16);
+        if (!FITS(p, 1) && FITS(v, 1)) p = v;
+    }
+#undef FITS
+    return p;
+}
+
 /* fixed_ws: NULL = the context's grow-only workspace; else the device's
  * fixed scratch of ORNK_SCRATCH_BYTES (gpu_moe_forward_noalloc), and the
  * call then allocates nothing. */
@@ -1233,29 +1259,15 @@ static int moe_forward_dev(gpu_context *ctx, ornith_moe_store *st, int layer, co
         use_mfma = 1;
     }
     if (file) use_mfma = 0;  /* the mid and combine steps run as on the VALU path */
-    plan_t p;
-    /* A store of blocks alone: the MFMA kernels that read them, unless the
-     * call forces the VALU kernels. */
-    int blk = !file && !mfma_ok && !(flags & ORN_MOE_PATH_VALU) && make_plan_blk(sh, T, &p);
-    if (!blk) p = file ? make_plan_file(sh, T) : make_plan(sh, T, use_mfma);
-
     /* Certified routing of the smallest decode batches (router_cert.hip):
      * logits, top-k and dispatch in one launch.  Streamed stores keep it too
      * (the slot list is read back after the dispatch either way). */
     const int cert = !(flags & ORN_MOE_EXACT_LOGITS) && ornk_route_cert_supported(T, D, E, k);
-
     const int norm = (flags & ORN_MOE_NORM) != 0;
-    if (blk) {
-        /* Its row maxima are a few bytes a row more than the VALU kernels'
-         * plan takes: at sizes where only that one fits the fixed scratch it
-         * runs, also in a call that may allocate (both give the same bits). */
-        const plan_t v = make_plan(sh, T, 0);
-        if (carve_ws(sh, T, &p, norm, cert, 1, ORNK_SYNC_BYTES).end > ORNK_SCRATCH_BYTES &&
-            carve_ws(sh, T, &v, norm, cert, 0, ORNK_SYNC_BYTES).end <= ORNK_SCRATCH_BYTES) {
-            blk = 0;
-            p = v;
-        }
-    }
+    /* A store of blocks alone: the MFMA kernels that read them, unless the
+     * call forces the VALU kernels. */
+    const plan_t p = choose_plan(sh, T, use_mfma, !mfma_ok && !(flags & ORN_MOE_PATH_VALU), norm, cert);
+    const int blk = p.use_blk;
 
     /* the fixed scratch keeps its first ORNK_SYNC_BYTES for the routing
      * counters (zeroed when the scratch is first resolved); otherwise they

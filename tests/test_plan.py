@@ -1,0 +1,48 @@
+"""The forward's plans (moe.c, built for the CPU by tests/plan_scan.c) over
+shapes and token counts: what a plan may not do, whatever it is chosen for."""
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def plans(tmp_path_factory):
+    exe = tmp_path_factory.mktemp("plan") / "plan_scan"
+    cmd = ["gcc", "-std=gnu99", "-O1", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-no-pie",
+           "-Wl,--unresolved-symbols=ignore-all", "-o", str(exe),
+           os.path.join(ROOT, "tests", "plan_scan.c"), "-lm"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-3000:]
+
+    def run(cases):
+        text = "\n".join(" ".join(map(str, c)) for c in cases)
+        out = subprocess.run([str(exe)], input=text, capture_output=True, text=True, check=True,
+                             timeout=300).stdout
+        return np.array([line.split() for line in out.splitlines()], int)
+    return run
+
+
+def shapes(rng, n):
+    E = rng.integers(1, 257, n)
+    k = np.minimum(rng.integers(1, 17, n), E)
+    T = np.exp(rng.uniform(0, np.log(4096), n)).astype(int)
+    return np.stack([rng.integers(0, 3, n), rng.choice([256, 512, 1024, 2048, 4096], n),
+                     rng.choice([256, 512, 1024], n), E, k, rng.integers(0, 2, n),
+                     rng.integers(0, 2, n), T], axis=1)
+
+
+def test_what_fits_the_fixed_scratch_is_not_refused(plans):
+    """No call is refused by gpu_moe_forward_noalloc for the plan it got where
+    another plan of the same products would fit."""
+    cases = shapes(np.random.default_rng(1), 200_000)
+    cases[0] = (0, 4096, 1024, 52, 2, 0, 0, 417)  # four tiles fit, two do not
+    cases[1] = (0, 2048, 512, 112, 15, 0, 0, 121)
+    got = plans(cases)
+    lost = cases[(got[:, 4] == 0) & (got[:, 5] == 1)]
+    assert not len(lost), lost[:10]
+    assert (got[:2, 4] == 1).all()
+
