@@ -1012,15 +1012,15 @@ static plan_t make_plan(const ornith_moe_shape *sh, int T, int use_mfma, int mos
             int dg = pow2_floor(ng > 0 ? ng : 1);
             while (dg > 1 && (D / 32) % dg) dg /= 2;
             while (dg > 1 && D / 32 / dg < 4) dg /= 2;
-            /* slices of 32 steps once two-tile items are many enough to fill
-             * the chip with half as many work groups: the mid step then reads
-             * half the partials (512 tokens gate/up 111 -> 105 us, mid 15 ->
-             * 10; 709: 124 -> 114 and 20 -> 13; 128 tokens of a skewed batch
-             * 34.0 -> 35.1 and 5.1 -> 4.4).  The whole layer with 16 steps /
-             * 32: 200 tokens 213.7 / 209.3 us, 256 219.9 / 215.8; skewed, whose
-             * few experts leave less to fill the chip with, 200 136.8 / 139.4,
-             * 256 130.6 / 132.4, 350 170.6 / 167.7. */
-            const int most = p.tchunk == 32 && T >= 192 ? 32 : 16;
+            /* Slices of 32 steps beyond 16 rows per expert, where the items
+             * are many enough to fill the chip with half as many work groups
+             * and the mid step then reads half the partials (512 tokens gate/up
+             * 111 -> 105 us, mid 15 -> 10; 709: 124 -> 114 and 20 -> 13).  Up
+             * to 16 rows uniform batches gain 2 % from it (200 tokens the
+             * layer 213.7 -> 209.3 us, 256 219.9 -> 215.8), but skewed ones,
+             * whose few experts leave less to fill the chip with, lose as much
+             * (200 136.8 -> 139.4, 256 130.6 -> 132.4), for sums twice as long. */
+            const int most = p.tchunk == 32 && T * k > 16 * E ? 32 : 16;
             while ((D / 32) % (2 * dg) == 0 && D / 32 / dg > most) dg *= 2;
             int dd = 1;
             while ((H / 32) % (2 * dd) == 0 && H / 32 / dd > 8) dd *= 2;

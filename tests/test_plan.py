@@ -46,3 +46,15 @@ def test_what_fits_the_fixed_scratch_is_not_refused(plans):
     assert not len(lost), lost[:10]
     assert (got[:2, 4] == 1).all()
 
+
+def test_gate_up_slices_of_thin_batches(plans):
+    """Up to 16 rows per expert a gate/up sum is at most 16 steps (512
+    products) long, unless the shape has no shorter slice."""
+    cases = shapes(np.random.default_rng(2), 100_000)
+    cases[:, 0] = 0
+    got = plans(cases)
+    T, E, k, D = (cases[:, i] for i in (7, 3, 4, 1))
+    thin = (got[:, 0] == 1) & (T * k <= 16 * E)
+    assert thin.sum() > 10_000
+    steps = D // 32 // got[:, 2]
+    assert (steps[thin] <= 16).all(), cases[thin][steps[thin] > 16][:10]
