@@ -21,6 +21,13 @@
 // row scales s are powers of two from the rows' max |x| and the slice's
 // largest |d|.
 //
+// Range: hi + lo hold a value to 2^-21 of itself down to 2^-17 of the row's and
+// slice's largest product, and to a fixed 2^-38 of that below.  What lies so far
+// down may be all that counts, where the weights of the rest are 0.  So a work
+// group that has such values and sums too small to hide them (SUM_MIN) goes
+// over its slice again for what hi + lo left out, times 2^24, and adds that to
+// what it stored; each pass reaches 2^24 further down.
+//
 // What bounds it: the vector instructions that form operands (gate/up about
 // 200 per wave and step for 36 MFMAs at two row tiles).  The fp32 matvec
 // kernels (expert_valu.hip) decode every weight once per token instead.
@@ -37,6 +44,7 @@ using namespace orn_mfma;
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 
+#define ORN_INLINE __attribute__((always_inline))
 #define ORN_BLK_KT 64  // most steps of a slice
 
 __device__ __forceinline__ rsrc_t make_rsrc(const void *p, uint32_t bytes)
@@ -73,6 +81,7 @@ struct BlkLds {
     float d[ORN_BLK_KT * 32];
     float scale[16 * RT], inv[16 * RT];
     float red[2];
+    uint32_t least[16 * RT];  // per row
 };
 
 // The largest v of the work group's 128 threads, in every one of them.
@@ -85,14 +94,106 @@ __device__ __forceinline__ float group_max(float v, float *red)
     return fmaxf(red[0], red[1]);
 }
 
-// VPT values of one row times d, hi/lo into the row's LDS words.
-template <int VPT>
-__device__ __forceinline__ void store_split(const float *x, const float *d, _Float16 *hi,
-                                            _Float16 *lo)
+// Whether some thread of the work group says so.
+__device__ __forceinline__ bool group_any(bool v, float *red)
 {
+    const float w = __any(v) ? 1.0f : 0.0f;
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = w;
+    __syncthreads();
+    const bool any = red[0] + red[1] > 0.0f;
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(any);
+}
+
+// The smallest magnitude but 0 that a thread has split, as bits.
+struct Least {
+    uint32_t v = ~0u;
+
+    static __device__ __forceinline__ uint32_t key(float x) { return 2 * __float_as_uint(x) - 1; }
+
+    template <int VPT>
+    __device__ __forceinline__ void see(const float (&a)[VPT])
+    {
+#pragma unroll
+        for (int i = 0; i < VPT; ++i) v = min(v, key(a[i]));
+    }
+};
+
+// Whether pass n over the rest has something to add to a row whose least is v:
+// the first has of values below 2^-3, the others of those another 2^24 down
+// (the fifth starts at 2^-99, where scaled operands begin to lack bits).
+__device__ __forceinline__ bool rest_of(uint32_t v, int n)
+{
+    return n <= 5 && v < Least::key(0x1p-3f) - ((uint32_t)(24 * (n - 1)) << 24);
+}
+
+constexpr float REST_UP = 0x1p24f;
+
+// 2^(-24 n)
+__device__ __forceinline__ float rest_scale(int n) { return __uint_as_float((uint32_t)(127 - 24 * n) << 23); }
+
+// Sums below which that may count: at 2^8 it is some 2^-21 of the sum (2^-26
+// per value, times weights of 2^8, 512 of them).  The largest of a thread's
+// eight sums of a row is compared: sums of ordinary operands are about 2^23 and
+// one of them may well be small, and a work group that goes over its slice
+// again can hold up the launch (gate/up at 300 tokens 147 us; 178 with every
+// sum compared by itself).  A row's sums alone decide what is added to them,
+// whatever the item's other rows are.
+constexpr float SUM_MIN = 0x1p8f;
+
+__device__ __forceinline__ float max8(const v4f (&s)[2])
+{
+    float m = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) m = fmaxf(m, fmaxf(fabsf(s[0][j]), fabsf(s[1][j])));
+    return m;
+}
+
+// Pass n over a row whose least is v, for the eight sums of one thread (pass
+// 0: s; later ones: what those before stored, old, to which s is added where
+// it may count).  lim = SUM_MIN in the sums' scale.  Whether another pass may
+// count.
+template <bool REST>
+__device__ __forceinline__ bool add_rest(v4f (&s)[2], const v4f (&old)[2], int n, uint32_t v, float lim)
+{
+    if constexpr (REST) {
+        const bool on = rest_of(v, n) && max8(old) < lim * rest_scale(n - 1);
+        const float f = rest_scale(n);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) s[h] = on ? old[h] + s[h] * f : old[h];
+        lim *= f;
+    }
+    return rest_of(v, n + 1) && max8(s) < lim;
+}
+
+// What hi + lo of split2 leave out of a, times 2^24; 0 where that is below
+// 2^-21 of a.
+__device__ __forceinline__ float split_rest(float a)
+{
+    if (!(fabsf(a) < 0.125f)) return 0.0f;
+    const v2h h = __builtin_bit_cast(v2h, __builtin_amdgcn_cvt_pkrtz(a, 0.0f));
+    const float r = a - (float)h.x;
+    const v2h l = __builtin_bit_cast(v2h, __builtin_amdgcn_cvt_pkrtz(r, 0.0f));
+    return (r - (float)l.x) * REST_UP;
+}
+
+// VPT values of one row times d (REST: what the passes before left out of that),
+// hi/lo into the row's LDS words.
+template <int VPT, bool REST>
+__device__ __forceinline__ void store_split(const float *x, const float *d, int pass, Least &least,
+                                            _Float16 *hi, _Float16 *lo)
+{
+    float a[VPT];
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) a[i] = x[i] * d[i];
+    if constexpr (!REST) least.see<VPT>(a);
+    else
+        for (int n = 0; n < pass; ++n)
+#pragma unroll
+            for (int i = 0; i < VPT; ++i) a[i] = split_rest(a[i]);
     uint32_t h[VPT / 2], l[VPT / 2];
 #pragma unroll
-    for (int i = 0; i < VPT / 2; ++i) split2(x[2 * i] * d[2 * i], x[2 * i + 1] * d[2 * i + 1], h[i], l[i]);
+    for (int i = 0; i < VPT / 2; ++i) split2(a[2 * i], a[2 * i + 1], h[i], l[i]);
     if constexpr (VPT == 8) {
         *reinterpret_cast<uint4 *>(hi) = make_uint4(h[0], h[1], h[2], h[3]);
         *reinterpret_cast<uint4 *>(lo) = make_uint4(l[0], l[1], l[2], l[3]);
@@ -107,24 +208,28 @@ __device__ __forceinline__ void store_split(const float *x, const float *d, _Flo
 // output gu[kslice][row][m*H + n].
 // ---------------------------------------------------------------------------
 template <int RT>
-__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(RT > 1 ? 2 : 3)))
-    k_gu_blk(const uint8_t *__restrict__ gate, const uint8_t *__restrict__ up,
-             const float *__restrict__ xn, const float *__restrict__ x_amax,
-             const int *__restrict__ ctl, const int4 *__restrict__ items,
-             const int *__restrict__ row_token, float *__restrict__ gu, int D, int H, int ks,
-             int rows_max)
+struct GuLds : BlkLds<RT, 4, 16> {  // S: 8 scales, 8 mins
+    float dm[ORN_BLK_KT * 32];
+};
+
+// Pass 0 over the slice, or (REST) a later one over what those before left out;
+// whether another is due.
+template <int RT, bool REST>
+__device__ __forceinline__ bool
+gu_pass(GuLds<RT> &L, int pass, int n_live, const uint8_t *__restrict__ gate,
+        const uint8_t *__restrict__ up, const float *__restrict__ xn,
+        const float *__restrict__ x_amax, const int4 *__restrict__ items,
+        const int *__restrict__ row_token, float *gu, int D, int H, int ks, int rows_max)
 {
-    constexpr int ROWS = 16 * RT, VPT = 4 * RT;
-    __shared__ __align__(16) BlkLds<RT, 4, 16> L;  // S: 8 scales, 8 mins
-    __shared__ __align__(16) float s_dm[ORN_BLK_KT * 32];
+    constexpr int VPT = 4 * RT;
     const int NB = H >> 8, per_item = 2 * NB * ks;
-    const int n_live = ctl[1] * per_item;
-    if ((int)blockIdx.x >= n_live) return;
     const int tile = xcd_remap(blockIdx.x, n_live);
     const int b = tile % NB, m = (tile / NB) & 1, kslice = (tile / (2 * NB)) % ks;
     const int4 itm = items[tile / per_item];
     const int e = itm.w, nrows = itm.z;
-    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
+    int tid = threadIdx.x;
+    if (REST) asm volatile("" : "+v"(tid));  // keeps nothing of pass 0's addresses
+    const int lane = tid & 63, g = lane >> 4, c = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int KT = D / 32 / ks, k0 = 32 * KT * kslice;
     const uint8_t *base =
@@ -140,7 +245,7 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(RT > 1
         uint32_t w[8];
         uint4 hd;
     } st0, st1;
-    auto load = [&](Ring &r, int kt) {
+    auto load = [&](Ring &r, int kt) ORN_INLINE {
         kt = kt < KT ? kt : KT - 1;
 #pragma unroll
         for (int i = 0; i < 8; ++i) r.w[i] = bload4(rq, w_off + i * ORN_Q4K_BYTES, kt * STEP);
@@ -156,7 +261,7 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(RT > 1
     struct XRow {
         float v[VPT];
     } x0, x1;
-    auto load_x = [&](XRow &x, int kt) {
+    auto load_x = [&](XRow &x, int kt) ORN_INLINE {
         kt = kt < KT ? kt : KT - 1;
 #pragma unroll
         for (int i = 0; i < VPT; i += 4) {
@@ -174,14 +279,16 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(RT > 1
         const uint32_t v = bload4(rq, (uint32_t)i * ORN_Q4K_BYTES, 0);
         const float d = orn_half_to_float(v & 0xFFFFu), dm = orn_half_to_float(v >> 16);
         L.d[i] = d;
-        s_dm[i] = dm;
+        L.dm[i] = dm;
         mx = fmaxf(mx, fmaxf(fabsf(d), fabsf(dm)));
     }
+    if (!REST && tid < 16 * RT) L.least[tid] = ~0u;
     mx = group_max(mx, L.red);
     const float as = live ? row_scale(x_amax[tok], mx) : 0.0f;
     if (ak == 0) L.inv[ar] = as != 0.0f ? 1.0f / as : 0.0f;
 
-    auto prep = [&](const uint4 &hd, const XRow &x, int kt, int buf) {
+    Least least;
+    auto prep = [&](const uint4 &hd, const XRow &x, int kt, int buf) ORN_INLINE {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             uint32_t sc, mn;
@@ -197,15 +304,12 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(RT > 1
             // results are not stored, but a NaN there must not be made)
             xs[i] = live ? x.v[i] * as : 0.0f;
             d[i] = L.d[32 * kt + ak + i];
-            dm[i] = s_dm[32 * kt + ak + i];
+            dm[i] = L.dm[32 * kt + ak + i];
         }
         const int o = ar * ORN_AST + ak;
-        store_split<VPT>(xs, d, &L.A[buf][0][o], &L.A[buf][1][o]);
-        store_split<VPT>(xs, dm, &L.A[buf][2][o], &L.A[buf][3][o]);
+        store_split<VPT, REST>(xs, d, pass, least, &L.A[buf][0][o], &L.A[buf][1][o]);
+        store_split<VPT, REST>(xs, dm, pass, least, &L.A[buf][2][o], &L.A[buf][3][o]);
     };
-    prep(st0.hd, x0, 0, 0);
-    load_x(x0, 2);
-    __syncthreads();
 
     v4f acc[RT][8], accm[RT];
 #pragma unroll
@@ -216,7 +320,7 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(RT > 1
     }
     const int rt_live = RT > 1 && nrows > 16 ? RT : 1;
 
-    auto sub = [&](Ring &st, const uint4 &nhd, XRow &nx, int kt, int buf) {
+    auto sub = [&](Ring &st, const uint4 &nhd, XRow &nx, int kt, int buf) ORN_INLINE {
         const uint4 slo = *reinterpret_cast<const uint4 *>(&L.S[buf][2 * ch][8 * g]);
         const uint4 shi = *reinterpret_cast<const uint4 *>(&L.S[buf][2 * ch + 1][8 * g]);
         uint4 mz = *reinterpret_cast<const uint4 *>(&L.S[buf][8 + 4 * wave + (c & 3)][8 * g]);
@@ -224,7 +328,7 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(RT > 1
         const v8h bm = __builtin_bit_cast(v8h, mz);
         const uint32_t sl[4] = {slo.x, slo.y, slo.z, slo.w}, sh[4] = {shi.x, shi.y, shi.z, shi.w};
         uint32_t o[8][4];
-        auto operand = [&](auto bbc) {
+        auto operand = [&](auto bbc) ORN_INLINE {
             constexpr int BB = decltype(bbc)::value;
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
@@ -265,12 +369,20 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(RT > 1
         load_x(nx, kt + 3);
         __syncthreads();
     };
+    prep(st0.hd, x0, 0, 0);
+    load_x(x0, 2);
+    __syncthreads();
     for (int kt = 0; kt < KT; kt += 2) {  // KT is even (launcher)
         sub(st0, st1.hd, x1, kt, 0);
         sub(st1, st0.hd, x0, kt + 1, 1);
     }
 
     const int col = m * H + 256 * b + 64 * ch + 4 * (di & 7);
+    bool again = false;
+    if constexpr (!REST) {
+        atomicMin(&L.least[ar], least.v);
+        __syncthreads();
+    }
     float *row0 = gu + ((size_t)kslice * rows_max + itm.y) * (2 * H) + col;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
@@ -281,17 +393,43 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(RT > 1
             const float ml = __shfl(accm[rt][r], 16 * g + 2 * (c >> 3), 64);
             const float mh = __shfl(accm[rt][r], 16 * g + 2 * (c >> 3) + 1, 64);
             if (row < nrows) {
-                v4f lo, hi;
+                v4f sum[2];
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    lo[j] = (acc[rt][j][r] - ml) * si;
-                    hi[j] = (acc[rt][4 + j][r] - mh) * si;
+                    sum[0][j] = (acc[rt][j][r] - ml) * si;
+                    sum[1][j] = (acc[rt][4 + j][r] - mh) * si;
                 }
                 float *o = row0 + (size_t)row * (2 * H);
-                *reinterpret_cast<v4f *>(o) = lo;
-                *reinterpret_cast<v4f *>(o + 32) = hi;
+                v4f old[2];
+                if constexpr (REST) {
+                    old[0] = *reinterpret_cast<const v4f *>(o);
+                    old[1] = *reinterpret_cast<const v4f *>(o + 32);
+                }
+                again = add_rest<REST>(sum, old, pass, L.least[row], SUM_MIN * si) || again;
+                *reinterpret_cast<v4f *>(o) = sum[0];
+                *reinterpret_cast<v4f *>(o + 32) = sum[1];
             }
         }
+    return group_any(again, L.red);
+}
+
+// (Two waves per SIMD: three leave 168 registers, with which the one-tile
+// instances spill.)
+template <int RT>
+__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
+    k_gu_blk(const uint8_t *__restrict__ gate, const uint8_t *__restrict__ up,
+             const float *__restrict__ xn, const float *__restrict__ x_amax,
+             const int *__restrict__ ctl, const int4 *__restrict__ items,
+             const int *__restrict__ row_token, float *gu, int D, int H, int ks, int rows_max)
+{
+    __shared__ __align__(16) GuLds<RT> L;
+    const int n_live = ctl[1] * 2 * (H >> 8) * ks;
+    if ((int)blockIdx.x >= n_live) return;
+    bool again = gu_pass<RT, false>(L, 0, n_live, gate, up, xn, x_amax, items, row_token, gu,
+                                    D, H, ks, rows_max);
+    for (int pass = 1; again; ++pass)
+        again = gu_pass<RT, true>(L, pass, n_live, gate, up, xn, x_amax, items, row_token, gu,
+                                  D, H, ks, rows_max);
 }
 
 // ---------------------------------------------------------------------------
@@ -303,22 +441,24 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(RT > 1
 // remainder operand (q6_b2's form).
 // ---------------------------------------------------------------------------
 template <int RT>
-__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(RT > 1 ? 2 : 3)))
-    k_dn_blk(const uint8_t *__restrict__ body, const uint16_t *__restrict__ dv,
-             const float *__restrict__ mid, const float *__restrict__ mid_amax,
-             const int *__restrict__ ctl, const int4 *__restrict__ items, float *__restrict__ dn,
-             int D, int H, int ks, int rows_max)
+using DnLds = BlkLds<RT, 2, 16>;
+
+template <int RT, bool REST>
+__device__ __forceinline__ bool
+dn_pass(DnLds<RT> &L, int pass, int n_live, const uint8_t *__restrict__ body,
+        const uint16_t *__restrict__ dv, const float *__restrict__ mid,
+        const float *__restrict__ mid_amax, const int4 *__restrict__ items, float *dn,
+        int D, int H, int ks, int rows_max)
 {
-    constexpr int ROWS = 16 * RT, VPT = 4 * RT;
-    __shared__ __align__(16) BlkLds<RT, 2, 16> L;
+    constexpr int VPT = 4 * RT;
     const int NB = D >> 8, per_item = NB * ks;
-    const int n_live = ctl[1] * per_item;
-    if ((int)blockIdx.x >= n_live) return;
     const int tile = xcd_remap(blockIdx.x, n_live);
     const int b = tile % NB, kslice = (tile / NB) % ks;
     const int4 itm = items[tile / per_item];
     const int e = itm.w, nrows = itm.z;
-    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
+    int tid = threadIdx.x;
+    if (REST) asm volatile("" : "+v"(tid));  // keeps nothing of pass 0's addresses
+    const int lane = tid & 63, g = lane >> 4, c = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int KT = H / 32 / ks, k0 = 32 * KT * kslice;
     const size_t blk0 = (size_t)(e * NB + b) * H + k0;
@@ -334,7 +474,7 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(RT > 1
     struct Ring {
         uint32_t l[8], q[8], sc;
     } st0, st1;
-    auto load = [&](Ring &r, int kt) {
+    auto load = [&](Ring &r, int kt) ORN_INLINE {
         kt = kt < KT ? kt : KT - 1;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -353,7 +493,7 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(RT > 1
     struct XRow {
         float v[VPT];
     } x0, x1;
-    auto load_x = [&](XRow &x, int kt) {
+    auto load_x = [&](XRow &x, int kt) ORN_INLINE {
         kt = kt < KT ? kt : KT - 1;
 #pragma unroll
         for (int i = 0; i < VPT; i += 4) {
@@ -371,11 +511,29 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(RT > 1
         L.d[i] = d;
         mx = fmaxf(mx, fabsf(d));
     }
+    if (!REST && tid < 16 * RT) L.least[tid] = ~0u;
     mx = group_max(mx, L.red);
-    const float as = live ? row_scale(mid_amax[arow], mx) : 0.0f;
+    // The row's largest in this slice: a saturated gate leaves slices whose
+    // values are all far below the row's largest, and so are their sums.
+    float xm = 0.0f;
+    if (ks == 1) {
+        xm = mid_amax[arow];
+    } else {
+#pragma unroll 4
+        for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+            for (int i = 0; i < VPT; i += 4) {
+                const v4f v = *reinterpret_cast<const v4f *>(xr + 32 * kt + i);
+                xm = fmaxf(fmaxf(xm, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+            }
+#pragma unroll
+        for (int o = 1; o < 32 / VPT; o *= 2) xm = fmaxf(xm, __shfl_xor(xm, o, 64));
+    }
+    const float as = live ? row_scale(xm, mx) : 0.0f;
     if (ak == 0) L.inv[ar] = as != 0.0f ? 1.0f / as : 0.0f;
 
-    auto prep = [&](uint32_t sc, const XRow &x, int kt, int buf) {
+    Least least;
+    auto prep = [&](uint32_t sc, const XRow &x, int kt, int buf) ORN_INLINE {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             L.S[buf][hj + i][hr] = (_Float16)(float)(int)(int8_t)(sc >> (8 * i));
@@ -387,11 +545,8 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(RT > 1
             d[i] = L.d[32 * kt + ak + i];
         }
         const int o = ar * ORN_AST + ak;
-        store_split<VPT>(xs, d, &L.A[buf][0][o], &L.A[buf][1][o]);
+        store_split<VPT, REST>(xs, d, pass, least, &L.A[buf][0][o], &L.A[buf][1][o]);
     };
-    prep(st0.sc, x0, 0, 0);
-    load_x(x0, 2);
-    __syncthreads();
 
     v4f acc[RT][8];
 #pragma unroll
@@ -400,7 +555,7 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(RT > 1
         for (int j = 0; j < 8; ++j) acc[rt][j] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
     const int rt_live = RT > 1 && nrows > 16 ? RT : 1;
 
-    auto sub = [&](Ring &st, uint32_t nsc, XRow &nx, int kt, int buf) {
+    auto sub = [&](Ring &st, uint32_t nsc, XRow &nx, int kt, int buf) ORN_INLINE {
         const int ro = c * ORN_AST + 8 * g;
         v8h ahi[RT], alo[RT];
 #pragma unroll
@@ -408,13 +563,13 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(RT > 1
             ahi[rt] = *reinterpret_cast<const v8h *>(&L.A[buf][0][16 * rt * ORN_AST + ro]);
             alo[rt] = *reinterpret_cast<const v8h *>(&L.A[buf][1][16 * rt * ORN_AST + ro]);
         }
-        auto half = [&](auto hic) {  // quarter `wave` (low nibbles), then wave + 2
+        auto half = [&](auto hic) ORN_INLINE {  // quarter `wave` (low nibbles), then wave + 2
             constexpr int HI = decltype(hic)::value;
             const uint4 s4 = *reinterpret_cast<const uint4 *>(&L.S[buf][sub_lo + 4 * HI][8 * g]);
             const uint32_t sv[4] = {s4.x, s4.y, s4.z, s4.w};
             const int sh = 2 * wave + 4 * HI;
             uint32_t o1[4][4], o2[4][4];
-            auto operand = [&](auto bbc) {
+            auto operand = [&](auto bbc) ORN_INLINE {
                 constexpr int BB = decltype(bbc)::value;
 #pragma unroll
                 for (int p = 0; p < 4; ++p) {
@@ -457,11 +612,19 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(RT > 1
         load_x(nx, kt + 3);
         __syncthreads();
     };
+    prep(st0.sc, x0, 0, 0);
+    load_x(x0, 2);
+    __syncthreads();
     for (int kt = 0; kt < KT; kt += 2) {
         sub(st0, st1.sc, x1, kt, 0);
         sub(st1, st0.sc, x0, kt + 1, 1);
     }
 
+    bool again = false;
+    if constexpr (!REST) {
+        atomicMin(&L.least[ar], least.v);
+        __syncthreads();
+    }
     float *row0 = dn + ((size_t)kslice * rows_max + itm.y) * D + 256 * b + 128 * n + 32 * wave + l4;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
@@ -470,17 +633,41 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(RT > 1
             const int row = 16 * rt + 4 * g + r;
             const float si = L.inv[row];
             if (row < nrows) {
-                v4f lo, hi;
+                v4f sum[2];
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    lo[j] = acc[rt][j][r] * si;
-                    hi[j] = acc[rt][4 + j][r] * si;
+                    sum[0][j] = acc[rt][j][r] * si;
+                    sum[1][j] = acc[rt][4 + j][r] * si;
                 }
                 float *o = row0 + (size_t)row * D;
-                *reinterpret_cast<v4f *>(o) = lo;
-                *reinterpret_cast<v4f *>(o + 64) = hi;
+                v4f old[2];
+                if constexpr (REST) {
+                    old[0] = *reinterpret_cast<const v4f *>(o);
+                    old[1] = *reinterpret_cast<const v4f *>(o + 64);
+                }
+                again = add_rest<REST>(sum, old, pass, L.least[row], SUM_MIN * si) || again;
+                *reinterpret_cast<v4f *>(o) = sum[0];
+                *reinterpret_cast<v4f *>(o + 64) = sum[1];
             }
         }
+    return group_any(again, L.red);
+}
+
+template <int RT>
+__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
+    k_dn_blk(const uint8_t *__restrict__ body, const uint16_t *__restrict__ dv,
+             const float *__restrict__ mid, const float *__restrict__ mid_amax,
+             const int *__restrict__ ctl, const int4 *__restrict__ items, float *dn, int D, int H,
+             int ks, int rows_max)
+{
+    __shared__ __align__(16) DnLds<RT> L;
+    const int n_live = ctl[1] * (D >> 8) * ks;
+    if ((int)blockIdx.x >= n_live) return;
+    bool again = dn_pass<RT, false>(L, 0, n_live, body, dv, mid, mid_amax, items, dn, D, H, ks,
+                                    rows_max);
+    for (int pass = 1; again; ++pass)
+        again = dn_pass<RT, true>(L, pass, n_live, body, dv, mid, mid_amax, items, dn, D, H, ks,
+                                  rows_max);
 }
 
 }  // namespace

@@ -33,14 +33,14 @@ def wide_scales(om, syn, seed):
     b[:, 192:208] = sc.astype(np.int8).view(np.uint8)
 
 
-def forward(om, ctx, st, x, flags, mode=0, names=None):
+def forward(om, ctx, st, x, flags, mode=0, names=None, resid=True):
     T, D = x.shape
     xb, ob = ctx.upload(x), ctx.alloc(x.nbytes)
     ib, wb = ctx.alloc(T * st.k * 4), ctx.alloc(T * st.k * 4)
     if names is not None:
         om.lib().gpu_profile_enable(ctx.ptr, 1)
         om.lib().gpu_profile_reset(ctx.ptr)
-    st.forward(0, xb, T, ob, resid=xb, idx=ib, w=wb, flags=flags, mode=mode)
+    st.forward(0, xb, T, ob, resid=xb if resid else None, idx=ib, w=wb, flags=flags, mode=mode)
     if names is not None:
         names += [n for n, (_, calls) in om.profile(ctx).items() if calls]
         om.lib().gpu_profile_enable(ctx.ptr, 0)
@@ -84,6 +84,55 @@ def test_blocks_mfma(om, ctx, D, H, E, k, wide, shared, T):
     assert np.allclose(w, rw, rtol=1e-5)
     assert row_err(out, ref) <= 1e-5 and row_err(valu, ref) <= 1e-5
     st.close()
+
+
+# Values that count 2^b below others whose weights are 0.
+#   x    x[0] = 2^b, gate and up rows 0 empty
+#   w    gate and up rows 0 with the largest d, x[0] = 0
+#   mid  x[1] = 2^b goes to the first 256 hidden values alone (gate row 1 is 1
+#        there and empty beyond), whose down rows are empty
+#   sparse  x[0] = 2^b as above, and two small values the only others
+# The bar is the other tests': fp32 arithmetic loses nothing here.
+@pytest.mark.parametrize("what,b", [("w", 0)] + [(w, b) for w in ("x", "mid", "sparse")
+                                                 for b in (0, 16, 20, 24, 30, 45, 60, 75)])
+@pytest.mark.parametrize("D,H,T", [(256, 512, 20), (2048, 512, 70), (1024, 1024, 3)])
+def test_blocks_mfma_wide_range(om, ctx, D, H, T, what, b):
+    E, k = 4, 2
+    syn = om.SyntheticLayer(D + H, 0, D, H, E, True)
+    wide_scales(om, syn, D)
+    x = om.synth_normal(T, om.synth_stream(0, om.SYN_ACT, 0), T * D, 1.0).reshape(T, D)
+    if what == "sparse":
+        x[:, :] = 0
+        x[:, [D // 2, D - 1]] = 1.5, -0.7
+    syn.router[:2] = 0
+    gate, up = (a.reshape(E + 1, D, H // 256, om.Q4K_BYTES) for a in (syn.gate, syn.up))
+    down = syn.down.reshape(E + 1, H, D // 256, om.Q6K_BYTES)
+    if what == "mid":
+        x[:, 0], x[:, 1] = 0, 2.0 ** b
+        up[:, 1] = 0
+        gate[:, 1] = 0
+        gate[:, 1, 0, :2] = np.float16(1).reshape(1).view(np.uint8)
+        gate[:, 1, 0, 4:8] = gate[:, 1, 0, 12:16] = 1  # scales 1, mins 0
+        gate[:, 1, 0, 16:] = 0x11
+        down[:, :256, :, 208:] = 0
+    elif what == "w":
+        x[:, 0] = 0
+        gate[:, 0, :, :4] = up[:, 0, :, :4] = np.float16([65504, 65504]).view(np.uint8)
+    else:
+        x[:, 0] = 2.0 ** b
+        gate[:, 0, :, :4] = up[:, 0, :, :4] = 0
+    st = om.Store(ctx, 1, D, H, E, k, True, prefill_layout=False)
+    st.load_layer(0, syn)
+    names = []
+    out, idx, _ = forward(om, ctx, st, x, 0, names=names, resid=False)
+    assert {"moe_gateup_blk", "moe_down_blk"} <= set(names)
+    valu, _, _ = forward(om, ctx, st, x, om.MOE_PATH_VALU, resid=False)
+    ref, ridx, _ = O.moe_layer(D=D, H=H, E=E, k=k, x=x, router_W=syn.router,
+                               gate=syn.routed("gate"), up=syn.routed("up"), down=syn.routed("down"),
+                               **{"sh_" + n: syn.shared(n) for n in ("gate", "up", "down")})
+    st.close()
+    assert np.array_equal(idx, ridx)
+    assert row_err(out, ref) <= 1e-5 and row_err(valu, ref) <= 1e-5
 
 
 def test_blocks_mfma_row_isolation(om, ctx):
