@@ -598,10 +598,23 @@ extern "C" int ornk_topk(const float *logits, int T, int E, int k, int mode, uin
 // ---------------------------------------------------------------------------
 // MoE routing step: exact logits into a->logits (selection: dispatch.hip).
 // ---------------------------------------------------------------------------
-extern "C" int ornk_router_pc_supported(int T, int D)
+extern "C" int ornk_router_pc_supported(int T, int E, int D)
 {
-    return T >= 1 && T <= ORN_ROUTER_PC_MAX_T &&
+    return T >= 1 && T <= ORN_ROUTER_PC_MAX_T && T * E <= ORN_ROUTER_PC_MAX_TE &&
            (D == 256 || D == 512 || D == 1024 || D == 2048 || D == 4096);
+}
+
+// One token per wave, its values broadcast by the multiplies, while that leaves
+// a SIMD few waves (the multiply takes twice the issue time, the LDS reads it
+// replaces are shared by every wave of the CU); then two, then four, broadcast
+// from LDS.  What counts is the work groups of one-token waves: four tokens by
+// 64 experts each, 2.5 and 6 per CU at the lines.  256 experts, us with one /
+// two / four: 300 tokens 29 / - / -, 512 32 / 37 / 52, 1000 54 / 45 / 56, 1500
+// 77 / 61 / 64, 2048 94 / 75 / 67.
+extern "C" int ornk_router_tpw(int T, int E)
+{
+    const int groups = ((E + 63) / 64) * ((T + 3) / 4);
+    return groups <= 640 ? 1 : groups <= 1536 ? 2 : 4;
 }
 
 extern "C" int ornk_moe_route(const ornk_moe_args *a, hipStream_t s)
@@ -614,7 +627,7 @@ extern "C" int ornk_moe_route(const ornk_moe_args *a, hipStream_t s)
     const float *xin = a->apply_norm ? a->xn : a->x;
     float *amax = a->router_amax ? a->x_amax : nullptr;  // every routing kernel can write it
     const dim3 gd((E + 7) / 8, T);
-    if (ornk_router_pc_supported(T, D)) {
+    if (ornk_router_pc_supported(T, E, D)) {
         // the norm runs inside the router here (ornk_moe_norm launches nothing)
         const float *xr = a->apply_norm ? a->x : xin;
         const float *nw = a->apply_norm ? a->norm_w : nullptr;
@@ -632,14 +645,7 @@ extern "C" int ornk_moe_route(const ornk_moe_args *a, hipStream_t s)
         }
 #undef ORN_RPC
     } else {
-        // Tokens per wave: one, their values broadcast by the multiplies,
-        // while that leaves a SIMD few waves (the multiply takes twice the
-        // issue time, the LDS reads it replaces are shared by every wave of
-        // the CU); then two, then four, broadcast from LDS.  us with one / two
-        // / four: 300 tokens 29 / - / -, 512 32 / 37 / 52, 1000 54 / 45 / 56,
-        // 1500 77 / 61 / 64, 2048 94 / 75 / 67.  (Up to 383 tokens each wave
-        // streamed the router from L2 before: 31 us at 65, 34 at 300.)
-        const int tpw = T < 640 ? 1 : T < 1536 ? 2 : 4;
+        const int tpw = ornk_router_tpw(T, E);
         const dim3 gs((E + 63) / 64, (T + 4 * tpw - 1) / (4 * tpw));
 #define ORN_RSEQ(TPW, NB)                                                                        \
     ORN_LAUNCH_EV(a, (k_router_seq<TPW, NB>), gs, dim3(256), 0, s, xin, a->router, a->bias, T, D, E, \

@@ -58,3 +58,17 @@ def test_gate_up_slices_of_thin_batches(plans):
     assert thin.sum() > 10_000
     steps = D // 32 // got[:, 2]
     assert (steps[thin] <= 16).all(), cases[thin][steps[thin] > 16][:10]
+
+
+def test_router_kernels_by_their_work():
+    """The routing kernels are chosen by the work they have (tokens times
+    experts), so that a layer of fewer experts keeps the faster ones to more
+    tokens: the one-token-per-group router up to 64 tokens, one token per wave
+    as long as four times the experts take a quarter of the tokens."""
+    import ornith_moe
+    pc, tpw = ornith_moe.lib().ornk_router_pc_supported, ornith_moe.lib().ornk_router_tpw
+    for E in (8, 64, 128, 176):
+        assert all(pc(t, E, 2048) for t in (1, 41, 64)) and not pc(65, E, 2048)
+    assert pc(44, 256, 2048) and not pc(45, 256, 2048) and not pc(64, 177, 2048)
+    for T in (4, 500, 640, 641, 1536, 1537, 4096):
+        assert tpw(T, 256) == tpw(2 * T, 128) == tpw(4 * T, 64) == tpw(4 * T, 8)

@@ -5,7 +5,8 @@ a sequential fp32 sum from 0 of the fp32 products x[d]*W[d*E+e], d
 ascending, then + bias), so the logits it selected on must equal the
 oracle's (oracle/oracle.c orc_router_logits) as uint32, for every kernel
 instance the forward picks:
-  - k_router_pc (T <= 40), with its fused rmsnorm when ORN_MOE_NORM is set;
+  - k_router_pc (up to 64 tokens and 11,264 logits), with its fused rmsnorm when
+    ORN_MOE_NORM is set;
   - k_router_seq (above, one, two or four tokens per wave), after the
     separate rmsnorm kernel;
 with and without a Zipf router bias, and for the file-orientation store
@@ -112,6 +113,27 @@ def check(om, ctx, store, T, layer, norm):
 @pytest.mark.parametrize("T", [1, 16, 64])
 def test_router_pc_logits_bit_exact(om, ctx, store, T, norm):
     check(om, ctx, store, T, 0, norm)
+
+
+# Fewer experts: the last logits of k_router_pc and the first beyond (176 and
+# 177 experts at 64 tokens), and the lines between one, two and four tokens per
+# wave where a row of experts takes one, two and three work groups.
+@pytest.mark.parametrize("E,T", [(64, 41), (128, 64), (176, 64), (177, 64), (200, 56), (64, 2560),
+                                 (40, 2561), (128, 1281), (128, 3073), (130, 2049)])
+def test_router_fewer_experts_logits_bit_exact(om, ctx, E, T):
+    d = 256
+    s = om.SyntheticLayer(E, 0, d, 256, E, False)
+    st = om.Store(ctx, 1, d, 256, E, K, False)
+    st.load_layer(0, s)
+    nw = (1.0 + 0.25 * np.random.default_rng(E).standard_normal(d)).astype(np.float32)
+    st.set_norm(0, nw)
+    x = om.synth_normal(T, om.synth_stream(0, om.SYN_ACT, 0), T * d, 1.0).reshape(T, d)
+    for norm in (False, True):
+        logits, idx, _ = forward(om, ctx, st, x, 0, (om.MOE_NORM if norm else 0) | om.MOE_EXACT_LOGITS)
+        ref = O.router_logits_rows(O.rmsnorm(x, nw) if norm else x, s.router, s.bias)
+        assert np.array_equal(logits.view(np.uint32), ref.view(np.uint32))
+        assert np.array_equal(idx, [O.topk(r, K, O.MODE_RENORM)[0] for r in ref])
+    st.close()
 
 
 @pytest.mark.parametrize("norm", [False, True], ids=["x", "rmsnorm"])
