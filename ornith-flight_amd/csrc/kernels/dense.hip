@@ -293,9 +293,11 @@ extern "C" int ornk_rmsnorm(float *out, const float *x, const float *w, int rows
     if (rows <= 0 || dim <= 0) return hipSuccess;
     if (dim > 16384) return hipErrorInvalidValue;  // the products live in LDS
     const bool al = (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) == 0;
-    // from two groups of rows on: below, the rows find a CU each (16 rows or
-    // 300 take the same time in groups of 8)
-    if (rows >= 2 * RN_R && dim % 32 == 0 && dim <= RN_MAXD && al && out != x) {
+    // Up to 512 rows a work group per row finds room on a CU beside one other,
+    // and its norm is the faster: dim 2048, 100 rows 13.4 us against 15.7, 256
+    // 13.6 / 16.4, 400 16.3 / 16.8, 600 23.0 / 16.9; dim 256 6.4 / 6.9, 6.5 / 7.3,
+    // 7.1 / 7.3, 9.0 / 7.3.
+    if (rows > 512 && dim % 32 == 0 && dim <= RN_MAXD && al && out != x) {
         hipLaunchKernelGGL(k_rmsnorm_rows, dim3((rows + RN_R - 1) / RN_R), dim3(256), 0, s, out, x,
                            w, rows, dim);
         return hipGetLastError();

@@ -144,16 +144,17 @@ def test_router_dec_logits_bit_exact(om, ctx, store, T, norm):
 
 @pytest.mark.parametrize("T", [384, 400, 1023, 1024, 2048])
 def test_router_seq_logits_bit_exact(om, ctx, store, T):
-    """LDS-staged chains: 4 tokens per block (T < 1024), 16 (T >= 1024)."""
+    """LDS-staged chains, four to sixteen tokens per work group."""
     check(om, ctx, store, T, 0, T == 400)
 
 
 @pytest.mark.parametrize("norm", [False, True], ids=["x", "rmsnorm"])
-@pytest.mark.parametrize("T", [40, 41, 43, 639, 640, 647, 1535, 1536])
+@pytest.mark.parametrize("T", [40, 41, 43, 44, 45, 512, 513, 639, 640, 641, 647, 1535, 1536, 1537])
 def test_router_instance_boundaries_bit_exact(om, ctx, store, T, norm):
-    """The step from the producer/consumer router to the staged one (40 / 41)
-    and between its instances of one, two and four tokens per wave, with work
-    groups whose last tokens are missing."""
+    """The step from the producer/consumer router to the staged one (44 / 45)
+    and between its instances of one, two and four tokens per wave (640 / 641,
+    1536 / 1537), with work groups whose last tokens are missing; with the norm,
+    the step to eight rows per work group (512 / 513) and a last group of seven."""
     check(om, ctx, store, T, 0, norm)
 
 
