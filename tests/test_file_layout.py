@@ -43,8 +43,9 @@ def file_plan(D, H, E, k, T):
     slots = min(T * k, E) + 1
     tchunk = 64 if T * k >= 16 * E else 16
     est = max(slots + rows // tchunk, 1)
-    kg = pow2_floor(max(8192 // (est * (2 * H // 256)), 1))
-    kd = pow2_floor(max(8192 // (est * (D // 128)), 1))
+    want = 2048 if tchunk == 64 else 8192
+    kg = pow2_floor(max(want // (est * (2 * H // 256)), 1))
+    kd = pow2_floor(max(want // (est * (D // 128)), 1))
     while kg > 1 and (D // 256) % kg:
         kg //= 2
     while kd > 1 and (H // 256) % kd:
@@ -345,12 +346,13 @@ def test_file_layout_shexp_gate(om, ctx, ornith_file, T):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("T,flags,mode", [(16, "norm", 0), (100, "norm", 0), (16, "", 1),
-                                          (100, "norm", 1)])
+                                          (100, "norm", 1), (40, "norm", 0), (41, "norm", 0),
+                                          (64, "norm", 0)])
 def test_file_layout_norm_resid_literal(om, ctx, ornith_file, T, flags, mode):
     """The call the engine integration makes (ORN_MOE_NORM with resid = x):
-    at T <= 64 the router's fused norm writes the normalised rows the
-    expert steps read, above that the separate norm kernel does; and the
-    literal routing mode (model.c:1027-1049)."""
+    up to 40 tokens (256 experts) the router's fused norm writes the normalised
+    rows and the file kernels' activations, above that a norm and a preparation
+    step of their own do; and the literal routing mode (model.c:1027-1049)."""
     D, H, E, k = 2048, 512, 256, 8
     syn, st = ornith_file
     rng = np.random.default_rng(50 + T + mode)
@@ -469,3 +471,61 @@ def test_file_layout_graph_replay_matches_eager(om, ctx, T):
         for b in (xb, ob, ib, wb):
             b.free()
         st.close()
+
+
+# One to four tokens at D >= 1024 run four launches: the certified router, which
+# writes the gate/up activations (and the rmsnorm), and a down kernel that forms
+# mid itself (four gate/up partials at D = 1024, eight at 2048).  Five tokens are
+# the first of the general path.
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,H", [(1024, 512), (2048, 512), (2048, 256)])
+@pytest.mark.parametrize("T", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("norm", [False, True], ids=["x", "rmsnorm"])
+@pytest.mark.parametrize("hot", [False, True], ids=["spread", "hot"])
+def test_file_layout_four_launches(om, ctx, D, H, T, norm, hot):
+    """hot: every token on the same experts, so that items hold T rows (the
+    shared expert's always do); Q6_K sub-scales over the int8 range; rows of
+    different size in one item.  By both routers, and by shares of the
+    experts, whose sum is the whole."""
+    E, k = 16, 8
+    syn = om.SyntheticLayer(D + H + T, 0, D, H, E, True)
+    rng = np.random.default_rng(T)
+    b = syn.down.reshape(-1, Q6K)
+    b[:, 192:208] = rng.integers(-128, 128, (b.shape[0], 16)).astype(np.int8).view(np.uint8)
+    x = rng.standard_normal((T, D)).astype(np.float32)
+    x[T // 2] *= 4
+    syn.router *= 0.1  # logits of order 1, whose roundings the weights do not show
+    if hot:
+        x[:, 0] = 3
+        syn.router[0, ::2] += 1
+    nw = (1.0 + 0.25 * rng.standard_normal(D)).astype(np.float32)
+    st = file_store(om, ctx, D, H, E, k, syn.gate, syn.up, syn.down, syn.router)
+    st.set_norm(0, nw)
+    kw = {"norm_w": nw, "resid": x} if norm else {}
+    ref, ridx, rw = oracle_file(syn, D, H, E, k, x, **kw)
+    if hot:
+        assert (np.sort(ridx, axis=1) == 2 * np.arange(k)).all()
+    L = om.lib()
+    for exact in (0, om.MOE_EXACT_LOGITS):
+        flags = (om.MOE_NORM if norm else 0) | exact
+        L.gpu_profile_enable(ctx.ptr, 1)
+        L.gpu_profile_reset(ctx.ptr)
+        out, idx, w = forward_full(ctx, st, x, k, flags=flags, resid=x if norm else None)
+        names = {n for n, (_, calls) in om.profile(ctx).items() if calls}
+        L.gpu_profile_enable(ctx.ptr, 0)
+        assert ("moe_mid" in names) == (T == 5), names
+        if not exact and T < 5:
+            assert names == {"moe_route", "moe_gateup_file", "moe_down_file", "moe_combine"}
+        assert np.array_equal(idx, ridx) and np.allclose(w, rw, rtol=1e-5, atol=1e-7)
+        assert row_err(out, ref).max() <= TOL
+    parts = np.zeros((T, D))
+    for ep in ((0, 5), (5, 11)):
+        xb, ob = ctx.upload(x), ctx.alloc(x.nbytes)
+        st.forward(0, xb, T, ob, flags=om.MOE_NORM if norm else 0, ep=ep)
+        parts += ctx.download(ob, np.float32, x.shape)
+        xb.free()
+        ob.free()
+    if norm:
+        parts += x
+    st.close()
+    assert row_err(parts, ref).max() <= TOL

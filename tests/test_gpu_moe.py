@@ -265,8 +265,8 @@ def test_mfma_residual_norm_and_row_independence(om, ctx, small):
 
 
 def test_mfma_needs_prefill_layout(om, ctx):
-    """Without the prefill layouts a large batch takes the VALU path, and
-    forcing the MFMA path is refused."""
+    """Without the prefill layouts a large batch takes the kernels that read the
+    blocks, and forcing the prefill layouts' MFMA path is refused."""
     L = Layer(om, ctx, 256, 256, 16, 8, seed=21, prefill_layout=False)
     x = act(om, 22, 150, 256)
     out, idx, _ = run(ctx, L, x)
