@@ -1386,7 +1386,7 @@ static int moe_forward_dev(gpu_context *ctx, ornith_moe_store *st, int layer, co
         /* the norm, logits, selection and dispatch in one launch */
         if ((rc = launch_k(ctx, "moe_route", ornk_moe_route_cert, &a))) return rc;
     } else {
-        if (a.apply_norm && !ornk_router_pc_supported(T, E, D) &&
+        if (a.apply_norm && !ornk_router_pc_supported(T, E, D, norm) &&
             (rc = launch(ctx, "moe_norm", ornk_moe_norm, &a)))
             return rc;
         if ((rc = launch_k(ctx, "moe_route", ornk_moe_route, &a))) return rc;
@@ -1397,7 +1397,7 @@ static int moe_forward_dev(gpu_context *ctx, ornith_moe_store *st, int layer, co
     if (st->cache && (rc = orn_cache_prepare(ctx, st->cache, layer, &a))) return rc;
     if (file) {
         /* decode sizes: the router wrote the file kernels' activations */
-        if (!cert && !ornk_router_pc_supported(T, E, D) &&
+        if (!cert && !ornk_router_pc_supported(T, E, D, norm) &&
             (rc = launch_k(ctx, "moe_file_prep_x", ornk_file_prep_x, &a)))
             return rc;
         if ((rc = launch_k(ctx, "moe_gateup_file", ornk_file_gateup, &a))) return rc;

@@ -223,16 +223,9 @@ typedef struct {
 
 int ornk_moe_norm(const ornk_moe_args *a, hipStream_t s);
 int ornk_moe_route(const ornk_moe_args *a, hipStream_t s);
-/* Batches the one-wave-per-(token, 8 experts) router takes (and that can
- * produce x_amax on the side). */
-/* Beyond, a separate norm and the staged router, whose 23.6 us (37 with the norm)
- * hardly grow up to 200 tokens.  This one's time is by its T * E / 8 work groups,
- * us without / with the norm: 256 experts 21.9 / 40.1 at 41 tokens, 22.7 / 41.9
- * at 48, 29.4 / 50.0 at 64; 128 experts 14.6 / 25.2 at 64, 64 experts 9.7 / 19.8.
- * The line, 40 tokens at 256 experts, lies between the two crossings. */
-#define ORN_ROUTER_PC_MAX_T 64
-#define ORN_ROUTER_PC_MAX_TE 10240
-int ornk_router_pc_supported(int T, int E, int D);
+/* Batches the one-wave-per-(token, 8 experts) router takes (norm: with the
+ * rmsnorm inside). */
+int ornk_router_pc_supported(int T, int E, int D, int norm);
 /* Tokens per wave of the staged router. */
 int ornk_router_tpw(int T, int E);
 /* Whether the decode down kernel forms mid itself (the mid step is then

@@ -598,19 +598,29 @@ extern "C" int ornk_topk(const float *logits, int T, int E, int k, int mode, uin
 // ---------------------------------------------------------------------------
 // MoE routing step: exact logits into a->logits (selection: dispatch.hip).
 // ---------------------------------------------------------------------------
-extern "C" int ornk_router_pc_supported(int T, int E, int D)
+// Its time is by its work groups, that of the staged router and a separate norm
+// hardly changes up to a few hundred tokens: the lines lie where they cross.  us
+// with 512 / 1024 / 1152 / 1536 / 2048 groups (256 experts, 16 to 64 tokens; the
+// same by 3 % at 64 experts), staged behind the bar:
+//   D = 1024   6.7 / 9.3 / 11.1 / 12.3 / 16.1 | 13.4
+//   D = 2048  10.2 / 14.6 / 20.8 / 22.7 / 28.8 | 22.2
+//   D = 4096    16 / 30 / 41 / 44 / 58 | 44
+// and with the norm
+//   D = 1024    11 / 14 / 14 / 16 / 22 | 24
+//   D = 2048    19 / 25 / 35 / 42 / 51 | 36
+//   D = 4096    37 / 67 / 86 / 95 / 124 | 67
+extern "C" int ornk_router_pc_supported(int T, int E, int D, int norm)
 {
-    return T >= 1 && T <= ORN_ROUTER_PC_MAX_T && T * E <= ORN_ROUTER_PC_MAX_TE &&
+    const int most = !norm ? 1536 : D <= 1024 ? 2048 : D <= 2048 ? 1152 : 1024;
+    return T >= 1 && (int64_t)T * ((E + 7) / 8) <= most &&
            (D == 256 || D == 512 || D == 1024 || D == 2048 || D == 4096);
 }
 
-// One token per wave, its values broadcast by the multiplies, while that leaves
-// a SIMD few waves (the multiply takes twice the issue time, the LDS reads it
-// replaces are shared by every wave of the CU); then two, then four, broadcast
-// from LDS.  What counts is the work groups of one-token waves: four tokens by
-// 64 experts each, 2.5 and 6 per CU at the lines.  256 experts, us with one /
-// two / four: 300 tokens 29 / - / -, 512 32 / 37 / 52, 1000 54 / 45 / 56, 1500
-// 77 / 61 / 64, 2048 94 / 75 / 67.
+// One token per wave, while that leaves a SIMD few waves; then two, then four.
+// What counts is the work groups of one-token waves, four tokens by 64 experts
+// each: 2.5 and 6 per CU at the lines.  256 experts, us with one / two / four:
+// 300 tokens 29 / - / -, 512 32 / 37 / 52, 1000 54 / 45 / 56, 1500 77 / 61 / 64,
+// 2048 94 / 75 / 67.
 extern "C" int ornk_router_tpw(int T, int E)
 {
     const int groups = ((E + 63) / 64) * ((T + 3) / 4);
@@ -627,7 +637,7 @@ extern "C" int ornk_moe_route(const ornk_moe_args *a, hipStream_t s)
     const float *xin = a->apply_norm ? a->xn : a->x;
     float *amax = a->router_amax ? a->x_amax : nullptr;  // every routing kernel can write it
     const dim3 gd((E + 7) / 8, T);
-    if (ornk_router_pc_supported(T, E, D)) {
+    if (ornk_router_pc_supported(T, E, D, a->apply_norm)) {
         // the norm runs inside the router here (ornk_moe_norm launches nothing)
         const float *xr = a->apply_norm ? a->x : xin;
         const float *nw = a->apply_norm ? a->norm_w : nullptr;
@@ -645,12 +655,17 @@ extern "C" int ornk_moe_route(const ornk_moe_args *a, hipStream_t s)
         }
 #undef ORN_RPC
     } else {
+        // One token per wave: its values are read from LDS while every work group
+        // has a CU (22.2 us at 100 tokens of 256 experts), and broadcast by the
+        // multiplies beyond, where the CU's waves share the LDS (which takes the
+        // multiplies twice the issue time: 23.6 at 100, 29.2 at 300).
         const int tpw = ornk_router_tpw(T, E);
         const dim3 gs((E + 63) / 64, (T + 4 * tpw - 1) / (4 * tpw));
 #define ORN_RSEQ(TPW, NB)                                                                        \
     ORN_LAUNCH_EV(a, (k_router_seq<TPW, NB>), gs, dim3(256), 0, s, xin, a->router, a->bias, T, D, E, \
                   a->logits, a->ctl, amax)
-        if (tpw == 1) ORN_RSEQ(1, 0);
+        if (tpw == 1 && gs.x * gs.y <= 256) ORN_RSEQ(1, 1);
+        else if (tpw == 1) ORN_RSEQ(1, 0);
         else if (tpw == 2) ORN_RSEQ(2, 1);
         else ORN_RSEQ(4, 4);
 #undef ORN_RSEQ

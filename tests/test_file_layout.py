@@ -346,11 +346,11 @@ def test_file_layout_shexp_gate(om, ctx, ornith_file, T):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("T,flags,mode", [(16, "norm", 0), (100, "norm", 0), (16, "", 1),
-                                          (100, "norm", 1), (40, "norm", 0), (41, "norm", 0),
+                                          (100, "norm", 1), (36, "norm", 0), (37, "norm", 0),
                                           (64, "norm", 0)])
 def test_file_layout_norm_resid_literal(om, ctx, ornith_file, T, flags, mode):
     """The call the engine integration makes (ORN_MOE_NORM with resid = x):
-    up to 40 tokens (256 experts) the router's fused norm writes the normalised
+    up to 36 tokens (256 experts) the router's fused norm writes the normalised
     rows and the file kernels' activations, above that a norm and a preparation
     step of their own do; and the literal routing mode (model.c:1027-1049)."""
     D, H, E, k = 2048, 512, 256, 8

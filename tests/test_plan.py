@@ -61,14 +61,17 @@ def test_gate_up_slices_of_thin_batches(plans):
 
 
 def test_router_kernels_by_their_work():
-    """The routing kernels are chosen by the work they have (tokens times
+    """The routing kernels are chosen by the work groups they have (tokens times
     experts), so that a layer of fewer experts keeps the faster ones to more
-    tokens: the one-token-per-group router up to 64 tokens, one token per wave
+    tokens: the one-token-per-group router up to 1536 groups of eight experts
+    (with the norm inside 2048, 1152 or 1024 by the width), one token per wave
     as long as four times the experts take a quarter of the tokens."""
     import ornith_moe
     pc, tpw = ornith_moe.lib().ornk_router_pc_supported, ornith_moe.lib().ornk_router_tpw
-    for E in (8, 64, 128, 160):
-        assert all(pc(t, E, 2048) for t in (1, 41, 64)) and not pc(65, E, 2048)
-    assert pc(40, 256, 2048) and not pc(41, 256, 2048) and not pc(64, 161, 2048)
+    for D, norm, most in ((256, 0, 1536), (2048, 0, 1536), (4096, 0, 1536), (1024, 1, 2048),
+                          (2048, 1, 1152), (4096, 1, 1024)):
+        for E in (8, 64, 128, 256):
+            assert pc(8 * most // E, E, D, norm) and not pc(8 * most // E + 1, E, D, norm)
+        assert pc(most // 2, 9, D, norm) and not pc(most // 2 + 1, 9, D, norm)
     for T in (4, 500, 640, 641, 1536, 1537, 4096):
         assert tpw(T, 256) == tpw(2 * T, 128) == tpw(4 * T, 64) == tpw(4 * T, 8)

@@ -5,7 +5,7 @@ a sequential fp32 sum from 0 of the fp32 products x[d]*W[d*E+e], d
 ascending, then + bias), so the logits it selected on must equal the
 oracle's (oracle/oracle.c orc_router_logits) as uint32, for every kernel
 instance the forward picks:
-  - k_router_pc (up to 64 tokens and 10,240 logits), with its fused rmsnorm when
+  - k_router_pc (up to 1536 groups of one token and eight experts), with its fused rmsnorm when
     ORN_MOE_NORM is set;
   - k_router_seq (above, one, two or four tokens per wave), after the
     separate rmsnorm kernel;
@@ -115,11 +115,12 @@ def test_router_pc_logits_bit_exact(om, ctx, store, T, norm):
     check(om, ctx, store, T, 0, norm)
 
 
-# Fewer experts: the last logits of k_router_pc and the first beyond (160 and
-# 161 experts at 64 tokens), and the lines between one, two and four tokens per
-# wave where a row of experts takes one, two and three work groups.
-@pytest.mark.parametrize("E,T", [(64, 41), (128, 64), (160, 64), (161, 64), (200, 52), (64, 2560),
-                                 (40, 2561), (128, 1281), (128, 3073), (130, 2049)])
+# Fewer experts: the last tokens of k_router_pc and the first beyond, without and
+# with the norm, and the lines between the staged instances where a row of
+# experts takes one, two and three work groups.
+@pytest.mark.parametrize("E,T", [(64, 41), (64, 192), (64, 193), (64, 256), (64, 257), (130, 120),
+                                 (40, 409), (40, 410), (128, 512), (128, 513), (64, 1024), (64, 1025),
+                                 (64, 2560), (40, 2561), (128, 1281), (128, 3073), (130, 2049)])
 def test_router_fewer_experts_logits_bit_exact(om, ctx, E, T):
     d = 256
     s = om.SyntheticLayer(E, 0, d, 256, E, False)
@@ -149,10 +150,10 @@ def test_router_seq_logits_bit_exact(om, ctx, store, T):
 
 
 @pytest.mark.parametrize("norm", [False, True], ids=["x", "rmsnorm"])
-@pytest.mark.parametrize("T", [40, 41, 43, 512, 513, 639, 640, 641, 647, 1535, 1536, 1537])
+@pytest.mark.parametrize("T", [36, 37, 40, 41, 43, 48, 49, 256, 257, 512, 513, 639, 640, 641, 647, 1535, 1536, 1537])
 def test_router_instance_boundaries_bit_exact(om, ctx, store, T, norm):
-    """The step from the producer/consumer router to the staged one (40 / 41)
-    and between its instances of one, two and four tokens per wave (640 / 641,
+    """The step from the producer/consumer router to the staged one (48 /
+    49, with the norm 36 / 37) and between its instances (256 / 257, 640 / 641,
     1536 / 1537), with work groups whose last tokens are missing; with the norm,
     the step to eight rows per work group (512 / 513) and a last group of seven."""
     check(om, ctx, store, T, 0, norm)
