@@ -152,7 +152,7 @@ def test_gpu_rope(om, ctx, hd, nq, nk, pos, theta):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("seq,hd", [(1, 64), (7, 256), (16, 128), (33, 80), (300, 256),
-                                    (1000, 64), (1500, 256), (513, 96), (65, 4), (5, 30),
+                                    (1000, 64), (1023, 64), (1024, 64), (1500, 256), (513, 96), (65, 4), (5, 30),
                                     (41, 18)])
 def test_gpu_attention(om, ctx, seq, hd):
     """Head dims that are a multiple of 4 run on the matrix cores (fp32
