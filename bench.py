@@ -372,9 +372,9 @@ def measure_streamed(ctx, steps):
 
 def measure_attention(ctx):
     """gpu_rope / gpu_attention (the Metal backend's semantics) at Ornith's
-    head size: one head, 4096 positions, head_dim 256, on the fp32 matrix
-    cores; 4*S^2*d flops per call against the MI355X dense fp32 peak
-    (157.3 TFLOP/s)."""
+    head size: one head, 4096 positions, head_dim 256.  At this length every
+    fp32 product is six products of bf16 parts, so the 4*S^2*d flops per call
+    are priced against a sixth of the MI355X dense bf16 peak (2.5 PFLOP/s)."""
     S, hd = 4096, 256
     rng = np.random.default_rng(0)
     bufs = [ctx.upload(rng.standard_normal((S, hd)).astype(np.float32)) for _ in range(3)]
@@ -396,8 +396,8 @@ def measure_attention(ctx):
     for b in bufs + [ob, q, k]:
         b.free()
     res = {"attention_s4096_d256": {"ms": round(dt * 1e3, 3), "tflops": round(tf, 2),
-                                    "bound": "mfma", "peak_fp32_tflops": 157.3,
-                                    "frac": round(tf / 157.3, 4)},
+                                    "bound": "mfma", "peak_tflops": round(2500 / 6, 1),
+                                    "frac": round(tf * 6 / 2500, 4)},
            "rope_16q2k_d256_us_per_call": round(rope_us, 2)}
     log("attention", res)
     return res

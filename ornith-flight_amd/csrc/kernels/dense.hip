@@ -4,8 +4,8 @@
 // forward.  Compiled with -ffp-contract=off: every mul/add below rounds
 // separately, in the order written, like the reference CPU backend
 // (gpu.c:104-156).  A code object of its own, loaded when one of them first
-// runs: as part of basic.hip's, which every context loads, its size cost the
-// one-token forward 0.5 us (25.5 -> 26.1) by where it left the others.
+// runs, and not part of basic.hip's, which every context loads: the one-token
+// forward moves by up to 0.5 us with what is loaded beside its kernels.
 #include "common.h"
 #include "launch.h"
 
@@ -193,7 +193,8 @@ __global__ void __launch_bounds__(256) k_rmsnorm(float *out, const float *x, con
 // the rows' chains side by side: a row's chain of dim dependent adds (5.8 us
 // at 2048) is what bounds it, and a work group per row keeps it for one lane.
 // 2048 rows of 2048: 48 -> 19 us, 1500 rows 37 -> 17 (event spans around the
-// launch, some 8 us of each their own).  dim % 32 == 0 and dim <= RN_MAXD.
+// launch, some 8 us of each their own).  dim % 32 == 0 and dim <= RN_MAXD, whose
+// eight rows take 66 KB of LDS: two work groups per CU, of 4096 columns one.
 constexpr int RN_MAXD = 2048, RN_R = 8;
 
 __global__ void __launch_bounds__(256) k_rmsnorm_rows(float *__restrict__ out,

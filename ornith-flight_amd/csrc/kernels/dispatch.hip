@@ -87,7 +87,9 @@ __device__ __forceinline__ void dispatch_keys(uint32_t (&ev)[ORN_DU], int p0, in
 // and written whole lines at a time.  One work group on one CU: what bounds it
 // is its memory instructions, above all the scattered four bytes per row
 // (2048 tokens, reading and counting twice and scattering to memory: 17.7 us;
-// 13.6 now).  NT = 0: any number of pairs, in that older way.
+// 13.6 now).  NT = 0: any number of pairs, in that older way (a third turn's
+// pairs would fit the LDS and the registers; larger batches than 2048 tokens of
+// top 8 were not measured with them).
 template <int NT, typename IdxT>
 __device__ void dispatch_group(DispatchLds &L, uint16_t *tok, const IdxT *sel_idx,
                                const float *sel_w, int T,

@@ -30,7 +30,8 @@
 //
 // What bounds it: the vector instructions that form operands (gate/up about
 // 200 per wave and step for 36 MFMAs at two row tiles).  The fp32 matvec
-// kernels (expert_valu.hip) decode every weight once per token instead.
+// kernels (expert_valu.hip) decode every weight once per token instead: 300
+// tokens 1216 us for the layer, here 283.
 #include "common.h"
 #include "launch.h"
 #include "mfma_ops.h"
