@@ -28,8 +28,8 @@
 // over its slice again for what hi + lo left out, times 2^24, and adds that to
 // what it stored; each pass reaches 2^24 further down.
 //
-// What bounds it: the vector instructions that form operands (gate/up about
-// 200 per wave and step for 36 MFMAs at two row tiles).  The fp32 matvec
+// What bounds it: the vector instructions that form operands (gate/up 264 per
+// wave and step for 18 MFMAs per row tile, down 372 for 24).  The fp32 matvec
 // kernels (expert_valu.hip) decode every weight once per token instead: 300
 // tokens 1216 us for the layer, here 283.
 #include "common.h"
