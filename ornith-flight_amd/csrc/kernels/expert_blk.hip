@@ -21,8 +21,8 @@
 // row scales s are powers of two from the rows' max |x| and the slice's
 // largest |d|.
 //
-// Range: hi + lo hold a value to 2^-21 of itself down to 2^-17 of the row's and
-// slice's largest product, and to a fixed 2^-38 of that below.  What lies so far
+// Range: hi + lo hold a value to 2^-23 of itself down to 2^-17 of the row's and
+// slice's largest product, and to a fixed 2^-39 of that below.  What lies so far
 // down may be all that counts, where the weights of the rest are 0.  So a work
 // group that has such values and sums too small to hide them (SUM_MIN) goes
 // over its slice again for what hi + lo left out, times 2^24, and adds that to
@@ -167,15 +167,26 @@ __device__ __forceinline__ bool add_rest(v4f (&s)[2], const v4f (&old)[2], int n
     return rest_of(v, n + 1) && max8(s) < lim;
 }
 
-// What hi + lo of split2 leave out of a, times 2^24; 0 where that is below
-// 2^-21 of a.
+// (a0, a1) -> hi and lo as in split2, but both rounded to nearest: 2^-23 of a
+// and no bias, where truncation leaves up to 2^-21 of one sign (one token's
+// error against 64 bits 2.7e-7 by the fp32 kernels, 6.8e-7 truncated).
+__device__ __forceinline__ void split2_rn(float a0, float a1, uint32_t &hi, uint32_t &lo)
+{
+    typedef float v2f __attribute__((ext_vector_type(2)));
+    const uint32_t h = as_u32(__builtin_convertvector((v2f){a0, a1}, v2h));
+    float r0, r1;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r0) : "v"(h), "v"(a0));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r1) : "v"(h), "v"(a1));
+    hi = h;
+    lo = as_u32(__builtin_convertvector((v2f){r0, r1}, v2h));
+}
+
+// What hi + lo leave out of a, times 2^24; 0 where that is below 2^-23 of a.
 __device__ __forceinline__ float split_rest(float a)
 {
     if (!(fabsf(a) < 0.125f)) return 0.0f;
-    const v2h h = __builtin_bit_cast(v2h, __builtin_amdgcn_cvt_pkrtz(a, 0.0f));
-    const float r = a - (float)h.x;
-    const v2h l = __builtin_bit_cast(v2h, __builtin_amdgcn_cvt_pkrtz(r, 0.0f));
-    return (r - (float)l.x) * REST_UP;
+    const float r = a - (float)(_Float16)a;
+    return (r - (float)(_Float16)r) * REST_UP;
 }
 
 // VPT values of one row times d (REST: what the passes before left out of that),
@@ -194,7 +205,7 @@ __device__ __forceinline__ void store_split(const float *x, const float *d, int 
             for (int i = 0; i < VPT; ++i) a[i] = split_rest(a[i]);
     uint32_t h[VPT / 2], l[VPT / 2];
 #pragma unroll
-    for (int i = 0; i < VPT / 2; ++i) split2(a[2 * i], a[2 * i + 1], h[i], l[i]);
+    for (int i = 0; i < VPT / 2; ++i) split2_rn(a[2 * i], a[2 * i + 1], h[i], l[i]);
     if constexpr (VPT == 8) {
         *reinterpret_cast<uint4 *>(hi) = make_uint4(h[0], h[1], h[2], h[3]);
         *reinterpret_cast<uint4 *>(lo) = make_uint4(l[0], l[1], l[2], l[3]);
