@@ -1076,8 +1076,11 @@ static plan_t make_plan_file(const ornith_moe_shape *sh, int T)
 /* MFMA kernels on vec@mat blocks: items of <= 16 rows up to 64 tokens, <= 32
  * above; the reduction is split so that gate/up and down have about 4096 work
  * groups of two waves (four rounds of the chip at their occupancy) but keep
- * slices of at least 4 steps, and no more partials than the VALU kernels'
- * plan (make_plan) where 64-step slices allow that, so that a batch that fits
+ * slices of at least 4 steps, gate/up at most 16 (sums half as long as 32 steps',
+ * which the fp32 kernels have here too, and 40 tokens 189 -> 174 us, Zipf
+ * batches of 40 / 65 / 300 108 / 128 / 188 -> 93 / 109 / 178, of 260 151 -> 154),
+ * and no more partials than the VALU kernels' plan (make_plan) where 64-step
+ * slices allow that, so that a batch that fits
  * the fixed scratch with that one fits with this one.  0 if the shape's slices are not taken. */
 static int make_plan_blk(const ornith_moe_shape *sh, int T, plan_t *out)
 {
@@ -1092,7 +1095,7 @@ static int make_plan_blk(const ornith_moe_shape *sh, int T, plan_t *out)
     const int est = max_slots + p.rows_max / p.tchunk;
     const int ng = 4096 / (est * (2 * H / 256)), nd = 4096 / (est * (D / 256));
     int kg = pow2_floor(ng > 0 ? ng : 1), kd = pow2_floor(nd > 0 ? nd : 1);
-    while (D / 32 / kg > 64) kg *= 2;
+    while (D / 32 / kg > 16) kg *= 2;
     while (kg > 1 && ((D / 32) % kg || D / 32 / kg < 4)) kg /= 2;
     while (kd > 1 && ((H / 32) % kd || H / 32 / kd < 4 || kd > 16)) kd /= 2;
     const plan_t v = make_plan(sh, T, 0, 0);
