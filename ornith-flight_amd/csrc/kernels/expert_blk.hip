@@ -28,10 +28,10 @@
 // over its slice again for what hi + lo left out, times 2^24, and adds that to
 // what it stored; each pass reaches 2^24 further down.
 //
-// What bounds it: the vector instructions that form operands (gate/up 264 per
+// What bounds it: the vector instructions that form operands (gate/up 278 per
 // wave and step for 18 MFMAs per row tile, down 372 for 24).  The fp32 matvec
 // kernels (expert_valu.hip) decode every weight once per token instead: 300
-// tokens 1216 us for the layer, here 283.
+// tokens 1216 us for the layer, here 273.
 #include "common.h"
 #include "launch.h"
 #include "mfma_ops.h"
