@@ -70,6 +70,8 @@
 #include <climits>
 #include <math.h>
 
+#include <type_traits>
+
 namespace {
 
 using namespace orn_sel;
@@ -92,8 +94,10 @@ struct CertArgs {
     int *ctl, *slot_expert, *slot_off, *slot_cnt, *row_token, *pair_row;
     int4 *items;
     int T, E, k, mode, ep_lo, ep_n, has_shared, items_max, tchunk;
-    int ngroups;  // expert work groups (with the rmsnorm or fx, one more group)
-    ornk_file_ws fx;  // file-orientation stores: the rows' hi/lo activations (xh NULL: none)
+    int ngroups;  // expert work groups (with the rmsnorm or FX, one more group)
+};
+struct CertFileArgs : CertArgs {
+    ornk_file_ws fx;  // file-orientation stores: the rows' hi/lo activations
 };
 
 __device__ __forceinline__ double readlane_d(double v, int l)
@@ -474,7 +478,7 @@ __device__ __forceinline__ int select_cert(float (&sfv)[4], float (&bfv)[4], boo
 }
 
 template <int NQ, bool FX>
-__global__ void __launch_bounds__(256) k_route_cert(CertArgs P)
+__global__ void __launch_bounds__(256) k_route_cert(std::conditional_t<FX, CertFileArgs, CertArgs> P)
 {
     constexpr int D = 256 * NQ, L = 4 * NQ;  // L: values per chunk (lane)
     __shared__ __align__(16) float xs[CERT_TPG][D];
@@ -834,7 +838,7 @@ extern "C" int ornk_moe_route_cert(const ornk_moe_args *a, hipStream_t s)
     if (a->ep_lo < 0 || a->ep_n < 0 || a->ep_lo + a->ep_n > E || !a->route_est || !a->sync)
         return hipErrorInvalidValue;
     if (T * a->k > ORN_CERT_MAX_T * 16 || a->tchunk < 1) return hipErrorInvalidValue;
-    CertArgs P;
+    CertFileArgs P;
     P.x = a->x;
     P.router = a->router;
     P.bias = a->bias;
@@ -864,14 +868,14 @@ extern "C" int ornk_moe_route_cert(const ornk_moe_args *a, hipStream_t s)
     P.tchunk = a->tchunk;
     P.ngroups = (E + CERT_EPG - 1) / CERT_EPG;
     P.fx = a->fw;
-    // a store of file blocks has instances of its own, so that the others'
-    // code stays as it is (one kernel for both measured 25.8 us for 25.6 at one
-    // token, which is near the spread of such runs)
+    // a store of file blocks has instances and arguments of its own, so that the
+    // others' stay as they are (one kernel for both measured 25.8 us for 25.6 at
+    // one token, which is near the spread of such runs)
     const bool fx = P.fx.xh != nullptr;
     const dim3 grid(P.ngroups + (P.norm_w || fx ? 1 : 0));  // + the extra group
 #define ORN_RC(N)                                                                        \
     if (fx) ORN_LAUNCH_EV(a, (k_route_cert<N, true>), grid, dim3(256), 0, s, P);         \
-    else ORN_LAUNCH_EV(a, (k_route_cert<N, false>), grid, dim3(256), 0, s, P)
+    else ORN_LAUNCH_EV(a, (k_route_cert<N, false>), grid, dim3(256), 0, s, static_cast<CertArgs &>(P))
     switch (D / 256) {
     case 1: ORN_RC(1); break;
     case 2: ORN_RC(2); break;
@@ -879,7 +883,7 @@ extern "C" int ornk_moe_route_cert(const ornk_moe_args *a, hipStream_t s)
     case 8: ORN_RC(8); break;
     case 16:  // file stores end at D = 2048
         if (fx) return hipErrorInvalidValue;
-        ORN_LAUNCH_EV(a, (k_route_cert<16, false>), grid, dim3(256), 0, s, P);
+        ORN_LAUNCH_EV(a, (k_route_cert<16, false>), grid, dim3(256), 0, s, static_cast<CertArgs &>(P));
         break;
     default: return hipErrorInvalidValue;
     }
